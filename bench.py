@@ -7,7 +7,11 @@ least-squares gradients with the Venkatakrishnan limiter, Roe flux, three
 Runge-Kutta stages per iteration, CFL 0.8 with local time stepping.  A step
 is one iteration of the reference's main loop (CCFVM/main.F90:57-128) on the
 device: primitive refresh, vertex averages, time step, gradient + limiter and
-three residual stages with their updates, then the residual norm.  Inputs are
+three residual stages with their updates, then the residual norm.  The
+reference refreshes the stages' inputs once per iteration, so the interior
+fluxes of the three stages are the same numbers; a whole iteration evaluates
+them once (the same results bit for bit) and `stage_by_stage` in the line
+gives the rate with every stage evaluating its whole residual.  Inputs are
 resident in HBM before the timed region.
 
 Metric: million cell-RK3-stages per second = 3 * cells * iterations / s / 1e6.
@@ -36,24 +40,24 @@ HBM_PEAK_GBS = 8000.0
 
 
 def stage_bytes(noc: int, nof: int, w: int, d: int = 8, i: int = 4) -> float:
-    """Algorithmic bytes of one residual-stage launch, averaged over the three
-    stages: face connectivity and geometry once per face, cell state once per
-    cell (primitives, gradients, limiter values, centroid), the old and the
-    current conserved state, dt/area, and the written state; the last stage
-    also writes the next iteration's primitives and temperature (5w per
-    cell, the primitive refresh it does for the next iteration)."""
+    """Algorithmic bytes of the residual pass of a whole RK3 iteration: face
+    connectivity and geometry once per face, cell data once per cell
+    (primitives, gradients, limiter values, centroid), the conserved state
+    read and written once, dt/area, and the next iteration's primitives and
+    temperature (5w per cell, the primitive refresh it does for the next
+    iteration).  One pass does all three stages: the reference's interior
+    fluxes are the same numbers in each (their inputs are refreshed once per
+    iteration), only the wall faces are evaluated per stage."""
     faces = nof * (2 * i + 5 * w)
-    cells = noc * (2 * w + 4 * w + 8 * w + 4 * w) + noc * 4 * d + noc * w + noc * 4 * d
-    prev_q = noc * 4 * d * 2.0 / 3.0
-    epilogue = noc * 5 * w / 3.0
-    return faces + cells + prev_q + epilogue
+    cells = noc * (2 * w + 4 * w + 8 * w + 4 * w) + noc * w + 2 * noc * 4 * d
+    return faces + cells + noc * 5 * w
 
 
 def pass_bytes(noc: int, nof: int, nop: int, nv2c: int, w: int, d: int = 8, i: int = 4) -> dict:
     """Algorithmic bytes per launch of the passes of a whole RK3 iteration, by
     profiling category: the vertex averages (P2), the face spectral radii
-    (P3), the gradient pass with the limiter and the time step (P4) and a
-    residual stage (P5, averaged over the three)."""
+    (P3), the gradient pass with the limiter and the time step (P4) and the
+    residual pass with the three stage updates (P5)."""
     p2 = nop * i + nv2c * (i + w) + noc * 4 * w + nop * 4 * w
     p3 = nof * (4 * i + 3 * w) + nop * 4 * w + noc * 2 * w
     p4 = nof * 2 * i + noc * (2 * w + 3 * w + 4 * w + 4 * w) + nof * 2 * w + noc * (8 * w + 4 * w)
@@ -61,23 +65,34 @@ def pass_bytes(noc: int, nof: int, nop: int, nv2c: int, w: int, d: int = 8, i: i
 
 
 def iteration_bytes(noc: int, nof: int, nop: int, nv2c: int, w: int, d: int = 8, i: int = 4) -> float:
-    """Algorithmic bytes of one RK3 iteration (all passes of the reference's
-    call structure: primitive refresh P1, vertex averages P2, spectral radii
-    P3, gradient and limiter P4, three residual stages P5)."""
-    p1 = noc * (4 * d + 4 * w)
-    p2 = nop * i + nv2c * (i + w) + noc * 4 * w + nop * 4 * w
-    p3 = nof * (4 * i + 3 * w) + nop * 4 * w + noc * 2 * w
-    p4 = nof * 2 * i + noc * (2 * w + 3 * w + 4 * w + 4 * w) + nof * 2 * w + noc * (8 * w + 4 * w)
-    faces = nof * (2 * i + 5 * w)
-    cells = noc * (2 * w + 4 * w + 8 * w + 4 * w) + noc * 4 * d + noc * w + noc * 4 * d
-    return p1 + p2 + p3 + p4 + 3 * (faces + cells) + 2 * noc * 4 * d
+    """Algorithmic bytes of one whole RK3 iteration: the sum of its passes."""
+    return sum(pass_bytes(noc, nof, nop, nv2c, w, d, i).values())
+
+
+def stage_by_stage(solver, steps: int, cfl: float = 0.8) -> float:
+    """Seconds of `steps` iterations driven routine by routine, as a host
+    program calls them, every stage evaluating its whole residual."""
+    def run(n):
+        for _ in range(n):
+            solver.prim()
+            solver.avg_c2v()
+            solver.time_step(cfl)
+            solver.save_old()
+            solver.gradient()
+            for k in (1, 2, 3):
+                solver.rk_stage(k)
+        solver.sync()
+    run(2)
+    t0 = time.perf_counter()
+    run(steps)
+    return time.perf_counter() - t0
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_stage_bump2M_hbm_traffic.md")
 
 
-STAGE_KERNELS = {"gather": ("k_stage", "false"), "gather_lds": ("k_stage", "true"),
-                 "shared": ("k_stage_blk", "false"), "shared_lds": ("k_stage_blk", "true")}
+STAGE_KERNELS = {"gather": ("k_rk3", "false"), "gather_lds": ("k_rk3", "true"),
+                 "shared": ("k_rk3_blk", "false"), "shared_lds": ("k_rk3_blk", "true")}
 
 
 def kernel_name(category: str, precision: str, form: str) -> str:
@@ -691,6 +706,7 @@ def main() -> int:
                   "frac": round(pbytes[k] / (kern[k] / 1000.0) / 1e9 / HBM_PEAK_GBS, 4)}
               for k in pbytes if k in kern}
 
+    by_stage = stage_by_stage(solver, args.steps)
     solver.close()
     # the mixed form (FP32 records, gradients, limiter and fluxes; FP64 state,
     # residual sums, time steps and norms) on the same mesh, timed the same
@@ -749,6 +765,10 @@ def main() -> int:
                      "avg_launch_ms": round(k_avg, 5)},
         "iteration_roofline_frac": round(it_bytes / (ms_step / 1000.0) / 1e9 / HBM_PEAK_GBS, 4),
         "passes": passes,
+        "stage_by_stage": {"value": round(3.0 * noc * args.steps / by_stage / 1e6, 2),
+                           "ms_per_step": round(by_stage * 1000.0 / args.steps, 4),
+                           "what": "routine by routine, every stage evaluating its whole "
+                                   "residual"},
         "stage_form": form,
         "stage_form_tuning": tune,
         **mixed,

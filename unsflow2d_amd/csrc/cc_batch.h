@@ -26,7 +26,7 @@ struct CaseDesc {
   double t_wall;
   double* hist;  // the context's residual history
   int iwall;
-  int nblk_all, nblk_pt, nblk_face, nblk_cell, nblk_bf;
+  int nblk_all, nblk_pt, nblk_face, nblk_cell, nblk_bc;
 };
 
 __device__ __forceinline__ VBlock case_block(const int4* map, int& c) {
@@ -54,14 +54,14 @@ __global__ __launch_bounds__(BLK) void km_prim(const CaseDesc<R>* cs, const int4
 
 // one block per case; the partials come from the primitive refresh (one
 // per block of all cells) or from the previous iteration's last stage (one
-// per block of interior cells)
+// per block of interior cells and of cells with boundary faces)
 template <typename R>
 __global__ __launch_bounds__(BLK) void km_range_final(const CaseDesc<R>* cs, const int4* map,
                                                       int from_stage) {
   int c;
   const VBlock vb = case_block(map, c);
   const CaseDesc<R> e = cs[c];
-  range_final_body<R>(e.d, vb, from_stage ? e.nblk_cell : e.nblk_all);
+  range_final_body<R>(e.d, vb, from_stage ? e.nblk_cell + e.nblk_bc : e.nblk_all);
 }
 
 template <typename R, bool VISC>
@@ -90,31 +90,31 @@ __global__ __launch_bounds__(BLK) void km_cell(const CaseDesc<R>* cs, const int4
 }
 
 template <typename R, int FLUX>
-__global__ __launch_bounds__(BLK) void km_bface(const CaseDesc<R>* cs, const int4* map,
-                                                int viscous_wall, int src) {
+__global__ __launch_bounds__(BLK) void km_rk3_bcell(const CaseDesc<R>* cs, const int4* map,
+                                                    int stored, int write_res, int epi) {
   int c;
   const VBlock vb = case_block(map, c);
   const CaseDesc<R> e = cs[c];
-  bface_body<R, FLUX>(e.d, vb, e.g, viscous_wall, e.iwall, e.t_wall, src);
+  rk3_bcell_body<R, FLUX>(e.d, vb, e.nblk_cell, e.gr, BndOpts{e.g, 0, e.iwall, e.t_wall},
+                          stored, write_res, epi);
 }
 
 template <typename R, int FLUX, bool SL>
-__global__ __launch_bounds__(BLK) void km_stage(const CaseDesc<R>* cs, const int4* map, int mode,
-                                                double ak, double bk, int write_res, int epi) {
+__global__ __launch_bounds__(BLK) void km_rk3(const CaseDesc<R>* cs, const int4* map, int rev,
+                                              int write_res, int epi) {
   int c;
-  const VBlock vb = case_block_dir(map, c, (mode & 16) != 0);
+  const VBlock vb = case_block_dir(map, c, rev != 0);
   const CaseDesc<R> e = cs[c];
-  stage_body<R, FLUX, SL>(e.d, vb, e.gr, mode, ak, bk, write_res, e.g, epi);
+  rk3_body<R, FLUX, SL>(e.d, vb, e.gr, e.g, rev, write_res, epi);
 }
 
 template <typename R, int FLUX, bool SL>
-__global__ __launch_bounds__(BLK) void km_stage_blk(const CaseDesc<R>* cs, const int4* map,
-                                                    int mode, double ak, double bk,
-                                                    int write_res, int epi) {
+__global__ __launch_bounds__(BLK) void km_rk3_blk(const CaseDesc<R>* cs, const int4* map, int rev,
+                                                  int write_res, int epi) {
   int c;
-  const VBlock vb = case_block_dir(map, c, (mode & 16) != 0);
+  const VBlock vb = case_block_dir(map, c, rev != 0);
   const CaseDesc<R> e = cs[c];
-  stage_blk_body<R, FLUX, SL>(e.d, vb, e.gr, mode, ak, bk, write_res, e.g, epi);
+  rk3_blk_body<R, FLUX, SL>(e.d, vb, e.gr, e.g, rev, write_res, epi);
 }
 
 // one block per case; history slot k of every case
@@ -123,7 +123,7 @@ __global__ void km_norm_final(const CaseDesc<R>* cs, const int4* map, int k) {
   int c;
   const VBlock vb = case_block(map, c);
   const CaseDesc<R> e = cs[c];
-  norm_final_body<R>(e.d, vb, e.nblk_cell, 0, e.hist, k);
+  norm_final_body<R>(e.d, vb, e.nblk_cell + e.nblk_bc, 0, e.hist, k);
 }
 
 // Per-variable residual norm of every case (as ufx_cc_residual_norm): block

@@ -14,8 +14,6 @@
 //   gT   [noc][2] R      its gradient (only when a consumer needs it)
 //   qc   [ncell][4] f64  conserved state [E, rho, rho u, rho v] (ghosts last)
 //   qold [noc][4] f64, res [noc][4] f64, dt/dta/la [noc] f64
-//   qs   [noc][4] f64    stage states of a whole RK3 iteration (qc keeps
-//                        the iteration's start state until the last stage)
 //   frec [nof][FW] R     face record nx, ny, area, centre x, y
 //   fcen [nof][2] R      face centre alone (for the gradient/limiter pass)
 //   fnl [nof][4] R       normal and length alone (for the face spectral radii)
@@ -69,7 +67,13 @@ struct DevT {
   const int2* fpt;
   const int* fbc;            // bc code per boundary ordinal (nbf)
   const int *bface, *bcell;  // storage face and inner cell per boundary ordinal
-  double* bres;              // [nbf][4] boundary-face fluxes of the current stage
+  double* bres;              // [nbf][4] boundary-face fluxes of a routine's residual
+  int nbc;                   // cells with boundary faces
+  const int* bc_cell;        // [nbc] those cells, ascending
+  const int* bc_ptr;         // per block of BLK cells, where its part of that list starts
+  R* bcF;                    // [MAXF][nbc][4] their interior fluxes (k_rk3_bcell)
+  const int4* bc_tab;        // [MAXF][nbc] per slot of those cells: sl_nbr, sl_face, kind of the
+                             // boundary face (0: interior face), cnf
   const int* sl_face;        // [MAXF][noc]
   const int* sl_nbr;         // [MAXF][noc]
   const int* cnf;            // nf | nb << 8
@@ -107,7 +111,6 @@ struct DevT {
   R* gT;
   double* qc;
   double* qold;
-  double* qs;                // [noc][4] stage states of whole RK3 iterations
   double* res;
   double* dt;
   double* dta;
@@ -275,7 +278,8 @@ struct OpAdd { __device__ double operator()(double a, double b) const { return a
 // names the face the reference's sequential loop would have stopped at:
 // Roe, key = boundary ordinal for boundary faces (looped first,
 // CCFVM/fvresidual.F90:27) and nbf + reference face for interior faces
-// (:133); diamond-path area, key = reference face.
+// (:133), plus (stage - 1) (nbf + nof) in a whole RK3 iteration; diamond-path
+// area, key = reference face.
 template <typename R>
 __device__ __forceinline__ void set_err(const DevT<R>& d, int code, int key) {
   int old = atomicCAS(d.err, 0, code);

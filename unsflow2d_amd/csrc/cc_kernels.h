@@ -638,25 +638,6 @@ __device__ __forceinline__ bool face_flux(const Gas<R>& g, R* ql, R* qr, R nx, R
   return true;
 }
 
-// Where a stage update reads and writes its states.  src 0 (routine by
-// routine): q = a qold + b (qc - dt/A R) in qc.  Whole RK3 iterations keep
-// the iteration's start state in qc and the stage states in qs, so no copy
-// to qold is needed: src 1 (stage 1) reads qc once and writes qs; src 2
-// (stage 2) reads qc and qs and writes qs; src 3 (stage 3) reads qc and qs
-// and writes qc (each cell reads only its own qc entry).
-template <typename R>
-__device__ __forceinline__ const double* stage_old(const DevT<R>& d, int src) {
-  return src ? d.qc : d.qold;
-}
-template <typename R>
-__device__ __forceinline__ const double* stage_in(const DevT<R>& d, int src) {
-  return src >= 2 ? d.qs : d.qc;
-}
-template <typename R>
-__device__ __forceinline__ double* stage_out(const DevT<R>& d, int src) {
-  return src == 1 || src == 2 ? d.qs : d.qc;
-}
-
 // The boundary conditions of a residual evaluation.
 struct BndOpts {
   Gas<double> g;
@@ -664,21 +645,21 @@ struct BndOpts {
   double t_wall;
 };
 
-// Boundary face k of a residual evaluation, CCFVM/fvresidual.F90:27-130, in
-// double: left state by the full-step reconstruction of the inner cell
+// Boundary face k (kind bc, storage face f) of a residual evaluation,
+// CCFVM/fvresidual.F90:27-130, in double: left state by the full-step reconstruction of the inner cell
 // (record `own`), farfield state or wall ghost (built from the inner cell's
-// current conserved state), flux F, ghost update and, for walls, the
-// momentum flux of the force sums.  F = 0 for other boundary kinds.
-template <typename R, int FLUX>
-__device__ __forceinline__ void bface_one(const DevT<R>& d, const BndOpts& bo, int k,
-                                          const R* own, int src, double* F) {
+// current conserved state, state(i)), flux F, ghost update and, for walls,
+// the momentum flux of the force sums.  F = 0 for other boundary kinds.
+// Returns false when the Roe average fails.
+template <typename R, int FLUX, typename State>
+__device__ __forceinline__ bool bface_one(const DevT<R>& d, const BndOpts& bo, int bc, int k,
+                                          int f, const R* own, State&& state, double* F) {
   constexpr int RW = Layout<R>::RW, FW = Layout<R>::FW;
   const Gas<double>& g = bo.g;
-  int bc = d.fbc[k];
 #pragma unroll
   for (int i = 0; i < 4; ++i) F[i] = 0.0;
-  if (bc != FARF && bc != WALL) return;
-  int f = d.bface[k], c = d.bcell[k], gh = d.noc + k;
+  if (bc != FARF && bc != WALL) return true;
+  int gh = d.noc + k;
   R fr[FW];
   face_rec(d, f, fr);
   double nx = fr[F_NX], ny = fr[F_NY], area = fr[F_AREA];
@@ -695,15 +676,18 @@ __device__ __forceinline__ void bface_one(const DevT<R>& d, const BndOpts& bo, i
     con2prim(g, gq, gp);
   } else {
     double q[4];
-    ld4d(stage_in(d, src) + (size_t)c * 4, q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = state(i);
     if (!bo.viscous_wall) {
-      // slip_wall, CCFVM/boundCond.F90:46-81
+      // slip_wall, CCFVM/boundCond.F90:46-81; its fused operations are spelt
+      // out, so that a routine's and a whole iteration's ghosts are the same
+      // bits however the compiler inlines them
       double rho = q[1], u = q[2] / q[1], v = q[3] / q[1];
-      double un = u * nx + v * ny;
+      double un2 = 2.0 * __builtin_fma(u, nx, v * ny);
       gq[0] = q[0];
       gq[1] = q[1];
-      gq[2] = rho * u - 2.0 * un * nx;
-      gq[3] = rho * v - 2.0 * un * ny;
+      gq[2] = __builtin_fma(rho, u, -(un2 * nx));
+      gq[3] = __builtin_fma(rho, v, -(un2 * ny));
       con2prim(g, gq, gp);
     } else if (bo.iwall == 1) {
       // adiabatic no-slip, CCFVM/boundCond.F90:31-37
@@ -731,32 +715,35 @@ __device__ __forceinline__ void bface_one(const DevT<R>& d, const BndOpts& bo, i
     d.bflux[k] = F[2];
     d.bflux[d.nbf + k] = F[3];
   }
-  if (!ok) set_err(d, DERR_ROE, k);
   st4d(d.qc + (size_t)gh * 4, gq);
   R gp4[4] = {(R)gp[0], (R)gp[1], (R)gp[2], (R)gp[3]};
   stv<R, 4>(d.rec + (size_t)gh * RW + R_QP, gp4);
   d.qT[gh] = (R)gp[4];
+  return ok;
 }
 
-// The boundary faces alone, one thread per face; the flux is stored for the
-// stage kernel, which adds it first, as the reference does.
+// The boundary faces of a routine's residual, one thread per face; the flux
+// is stored for the stage kernel, which adds it first, as the reference does.
 template <typename R, int FLUX>
 __device__ __forceinline__ void bface_body(const DevT<R>& d, VBlock vb, Gas<double> g,
-                                           int viscous_wall, int iwall, double t_wall, int src) {
+                                           int viscous_wall, int iwall, double t_wall) {
   constexpr int RW = Layout<R>::RW;
   int k = vb.b * BLK + threadIdx.x;
   if (k >= d.nbf || d.err[0]) return;
   const BndOpts bo{g, viscous_wall, iwall, t_wall};
+  const int c = d.bcell[k];
   R own[RW];
-  ldv<R, RW>(d.rec + (size_t)d.bcell[k] * RW, own);
+  ldv<R, RW>(d.rec + (size_t)c * RW, own);
   double F[4];
-  bface_one<R, FLUX>(d, bo, k, own, src, F);
+  if (!bface_one<R, FLUX>(d, bo, d.fbc[k], k, d.bface[k], own,
+                          [&](int i) { return d.qc[(size_t)c * 4 + i]; }, F))
+    set_err(d, DERR_ROE, k);
   st4d(d.bres + (size_t)k * 4, F);
 }
 template <typename R, int FLUX>
 __global__ __launch_bounds__(BLK) void k_bface(DevT<R> d, Gas<double> g, int viscous_wall,
-                                               int iwall, double t_wall, int src) {
-  bface_body<R, FLUX>(d, hw_block(), g, viscous_wall, iwall, t_wall, src);
+                                               int iwall, double t_wall) {
+  bface_body<R, FLUX>(d, hw_block(), g, viscous_wall, iwall, t_wall);
 }
 
 // Copy the records of the block's cells [base, base + cnt) into LDS with
@@ -786,10 +773,13 @@ __device__ __forceinline__ void load_rec(const DevT<R>& d, const R* srec, int ba
 // faces with recon (:190-252) on both sides, each flux evaluated from the
 // same inputs by both adjacent cells.  Returns the lowest failing face key
 // (set_err), INT_MAX when every flux succeeded.  SL: records of the block's
-// cells [base, base + BLK) are read from srec.
-template <typename R, int FLUX, bool SL>
+// cells [base, base + BLK) are read from srec.  BND = false: the interior
+// faces alone.  keep: where the interior fluxes are also stored, 4 values per
+// slot, `stride` values apart (null: nowhere).
+template <typename R, int FLUX, bool SL, bool BND = true>
 __device__ __forceinline__ int gather_residual(const DevT<R>& d, const R* srec, int base, int c,
-                                               const Gas<R>& gr, double* r) {
+                                               const Gas<R>& gr, double* r,
+                                               R* keep = nullptr, size_t stride = 0) {
   constexpr int RW = Layout<R>::RW, FW = Layout<R>::FW;
   const int noc = d.noc;
   int info = ld_nt(d.cnf + c), nf = info & 0xff, nb = info >> 8;
@@ -798,7 +788,7 @@ __device__ __forceinline__ int gather_residual(const DevT<R>& d, const R* srec, 
 #pragma unroll
   for (int i = 0; i < 4; ++i) r[i] = 0.0;
   int ekey = INT_MAX;
-  for (int s = nf - nb; s < nf; ++s) {
+  for (int s = nf - nb; BND && s < nf; ++s) {
     int k = ld_nt(d.sl_nbr + s * noc + c) - noc;
     double F[4];
     ld4d(d.bres + (size_t)k * 4, F);
@@ -844,6 +834,7 @@ __device__ __forceinline__ int gather_residual(const DevT<R>& d, const R* srec, 
     }
     if (!face_flux<R, FLUX>(gr, ql, qr, fr[F_NX], fr[F_NY], fr[F_AREA], F))
       ekey = min(ekey, d.nbf + d.fref[f]);
+    if (sizeof(R) == 4 && !BND && keep) stv<R, 4>(keep + s * stride, F);
     if (in_side) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) r[i] = r[i] + (double)F[i];
@@ -853,136 +844,6 @@ __device__ __forceinline__ int gather_residual(const DevT<R>& d, const R* srec, 
     }
   }
   return ekey;
-}
-
-// The primitive refresh of the next iteration (CCFVM/main.F90:62-67), done
-// by the last stage of a whole RK3 iteration from the state it has just
-// written, so that the next iteration needs no pass of its own for it: the
-// compact primitives and temperature qpc, qTc (the gradient pass copies them
-// into the records and qT, which this stage's other cells are still
-// gathering, and which stay the reference's qp until then), the
-// positivity note for the next iteration (err[1], moved up by the norm) and
-// the block's partial of the limiter's global range over its cells and the
-// ghosts of their boundary faces (written by this stage's k_bface).  Called
-// by every thread of the block; `have`: the thread's cell is interior and
-// its new state is q.
-template <typename R>
-__device__ __forceinline__ void prim_epilogue(const DevT<R>& d, VBlock vb, const Gas<double>& g,
-                                              int c, bool have, const double* q) {
-  constexpr int RW = Layout<R>::RW;
-  __shared__ double shr[8][BLK / 64];
-  double mx[4], mn[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) { mx[k] = -INFINITY; mn[k] = INFINITY; }
-  if (have) {
-    double p[5];
-    con2prim(g, q, p);
-    R q4[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) q4[k] = (R)p[k];
-    stv<R, 4>(d.qpc + (size_t)c * 4, q4);
-    d.qTc[c] = (R)p[4];
-    if (p[0] <= 0.0 || p[3] <= 0.0) atomicMin(&d.err[1], d.cref[c] + 1);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) mx[k] = mn[k] = (double)q4[k];
-    const int info = ld_nt(d.cnf + c), nf = info & 0xff, nb = info >> 8;
-    for (int s = nf - nb; s < nf; ++s) {
-      const int gh = ld_nt(d.sl_nbr + s * d.noc + c);
-      R gq[4];
-      ldv<R, 4>(d.rec + (size_t)gh * RW + R_QP, gq);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const double v = (double)gq[k];
-        mx[k] = v > mx[k] ? v : mx[k];
-        mn[k] = v < mn[k] ? v : mn[k];
-      }
-    }
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      double a = __shfl_xor(mx[k], off), b = __shfl_xor(mn[k], off);
-      mx[k] = a > mx[k] ? a : mx[k];
-      mn[k] = b < mn[k] ? b : mn[k];
-    }
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  if (lane == 0)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      shr[k][wave] = mx[k];
-      shr[4 + k][wave] = mn[k];
-    }
-  __syncthreads();
-  if (threadIdx.x < 8) {
-    const int k = threadIdx.x;
-    double a = shr[k][0];
-    for (int w = 1; w < BLK / 64; ++w)
-      a = k < 4 ? (shr[k][w] > a ? shr[k][w] : a) : (shr[k][w] < a ? shr[k][w] : a);
-    d.rpart[(size_t)vb.b * 8 + k] = a;
-  }
-}
-
-// Residual stage over the block's cells (gather_residual), then
-//   mode & 3 = 0: store the residual only;
-//              1: apply the stage update of CCFVM/main.F90:92-101 (no other
-//                 cell reads this cell's state during a stage);
-//              2: 1 and a block partial of the squared residual;
-//   (mode >> 2) & 3 (src): where the update's states live, stage_old/in/out;
-//   mode & 16: the XCDs walk their slices of blocks from the far end.
-// SL: the block's records are first copied to LDS, so the neighbours inside
-// the block (most of them, the cells being Hilbert-ordered) are read from
-// there instead of through L2.  epi: the last stage of a whole iteration
-// also refreshes the primitives (prim_epilogue).
-template <typename R, int FLUX, bool SL>
-__device__ __forceinline__ void stage_body(const DevT<R>& d, VBlock vb, Gas<R> gr, int mode,
-                                           double ak, double bk, int write_res,
-                                           const Gas<double>& g, int epi) {
-  const int op = mode & 3, src = (mode >> 2) & 3;
-  const bool rev = (mode & 16) != 0;
-  extern __shared__ double lds_raw[];
-  R* srec = reinterpret_cast<R*>(lds_raw);  // [BLK][RW] when SL
-  __shared__ double sh[1][BLK];
-  const int base = xcd_block_dir(vb.b, vb.n, rev) * BLK;
-  const int c = base + threadIdx.x;
-  if (SL) {
-    stage_block_recs(d, srec, base, min(BLK, d.noc - base));
-    __syncthreads();
-  }
-  double sq = 0.0, q[4] = {0.0, 0.0, 0.0, 0.0};
-  bool have = false;
-  if (c < d.noc && !d.err[0]) {
-    double r[4];
-    const int ekey = gather_residual<R, FLUX, SL>(d, srec, base, c, gr, r);
-    if (ekey != INT_MAX) set_err(d, DERR_ROE, ekey);
-    if (op == 0 || write_res) st4d_nt(d.res + (size_t)c * 4, r);
-    if (op >= 1) {
-      double dta = ld_nt(d.dta + c), o[4];
-      ld4d_nt(stage_old(d, src) + (size_t)c * 4, o);
-      if (src == 1) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) q[i] = o[i];
-      } else {
-        ld4d_nt(stage_in(d, src) + (size_t)c * 4, q);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) q[i] = rk_update1(ak, o[i], bk, q[i], dta, r[i]);
-      st4d_nt(stage_out(d, src) + (size_t)c * 4, q);
-      have = true;
-    }
-    if (op == 2)
-      for (int i = 0; i < 4; ++i) sq = sq + r[i] * r[i];
-  }
-  if (op == 2) {
-    block_reduce<1>(sh, &sq, OpAdd());
-    if (threadIdx.x == 0) d.part[vb.b] = sq;
-  }
-  if (epi) prim_epilogue<R>(d, vb, g, c, have, q);
-}
-template <typename R, int FLUX, bool SL>
-__global__ __launch_bounds__(BLK) void k_stage(DevT<R> d, Gas<R> gr, int mode, double ak, double bk,
-                                               int write_res, Gas<double> g, int epi) {
-  stage_body<R, FLUX, SL>(d, hw_block(), gr, mode, ak, bk, write_res, g, epi);
 }
 
 // Flux through interior face `f` from the records of its `in` cell (a) and
@@ -1008,35 +869,337 @@ __device__ __forceinline__ bool face_flux_ab(const Gas<R>& gr, const R* ra, cons
   return face_flux<R, FLUX>(gr, ql, qr, fr[F_NX], fr[F_NY], fr[F_AREA], F);
 }
 
-// The residual stage of k_stage with every interior flux evaluated once per
-// block instead of once per adjacent cell.  Phase 1: the block's threads
-// walk the interior faces touched by its BLK cells (Hilbert-ordered, so
-// about 1.65 faces per cell instead of 3), evaluate each flux once and keep
-// it in LDS.  Phase 2: each cell sums the boundary fluxes and then its
-// interior fluxes from LDS in its slot order (the reference's accumulation
-// order), then applies the stage update as k_stage does.  SL as in k_stage.
+// The end of a routine-by-routine stage of cell c with residual r.
+template <typename R>
+__device__ __forceinline__ void stage_end(const DevT<R>& d, int c, int op, double ak, double bk,
+                                          int write_res, const double* r) {
+  if (op == 0 || write_res) st4d_nt(d.res + (size_t)c * 4, r);
+  if (op == 1) {
+    double dta = ld_nt(d.dta + c), o[4], q[4];
+    ld4d_nt(d.qold + (size_t)c * 4, o);
+    ld4d_nt(d.qc + (size_t)c * 4, q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = rk_update1(ak, o[i], bk, q[i], dta, r[i]);
+    st4d_nt(d.qc + (size_t)c * 4, q);
+  }
+}
+
+// The end of a block of a whole RK3 iteration: the block's partial of the
+// squared residual (slot `slot` of part), and with epi the primitive refresh
+// of the next iteration (CCFVM/main.F90:62-67) from the state just written,
+// so that the next iteration needs no pass of its own for it: the
+// compact primitives and temperature qpc, qTc (the gradient pass copies them
+// into the records and qT, which other cells are still gathering, and which
+// stay the reference's qp until then), the positivity note for the next
+// iteration (err[1], moved up by the norm) and the block's partial of the
+// limiter's global range over its cells and, with GHOSTS, the ghosts of
+// their boundary faces (which the same thread has written).  Called by every
+// thread of the block; `have`: the thread's cell c is interior, its new state
+// is q and its squared residual sq.
+template <typename R, bool GHOSTS>
+__device__ __forceinline__ void rk3_finish(const DevT<R>& d, int slot, const Gas<double>& g, int c,
+                                           bool have, const double* q, double sq, int epi) {
+  constexpr int RW = Layout<R>::RW;
+  __shared__ double shr[9][BLK / 64];
+  double mx[4], mn[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) { mx[k] = -INFINITY; mn[k] = INFINITY; }
+  if (have && epi) {
+    double p[5];
+    con2prim(g, q, p);
+    R q4[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) q4[k] = (R)p[k];
+    stv<R, 4>(d.qpc + (size_t)c * 4, q4);
+    d.qTc[c] = (R)p[4];
+    if (p[0] <= 0.0 || p[3] <= 0.0) atomicMin(&d.err[1], d.cref[c] + 1);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mx[k] = mn[k] = (double)q4[k];
+    if (GHOSTS) {
+      const int info = ld_nt(d.cnf + c), nf = info & 0xff, nb = info >> 8;
+      for (int s = nf - nb; s < nf; ++s) {
+        const int gh = ld_nt(d.sl_nbr + s * d.noc + c);
+        R gq[4];
+        ldv<R, 4>(d.rec + (size_t)gh * RW + R_QP, gq);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const double v = (double)gq[k];
+          mx[k] = v > mx[k] ? v : mx[k];
+          mn[k] = v < mn[k] ? v : mn[k];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    sq = sq + __shfl_xor(sq, off);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double a = __shfl_xor(mx[k], off), b = __shfl_xor(mn[k], off);
+      mx[k] = a > mx[k] ? a : mx[k];
+      mn[k] = b < mn[k] ? b : mn[k];
+    }
+  }
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  if (lane == 0) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      shr[k][wave] = mx[k];
+      shr[4 + k][wave] = mn[k];
+    }
+    shr[8][wave] = sq;
+  }
+  __syncthreads();
+  if (threadIdx.x < 9) {
+    const int k = threadIdx.x;
+    double a = shr[k][0];
+    for (int w = 1; w < BLK / 64; ++w) {
+      const double b = shr[k][w];
+      a = k == 8 ? a + b : k < 4 ? (b > a ? b : a) : (b < a ? b : a);
+    }
+    if (k == 8) d.part[slot] = a;
+    else if (epi) d.rpart[(size_t)slot * 8 + k] = a;
+  }
+}
+
+// Residual stage over the block's cells (gather_residual), routine by
+// routine: store the residual (op 0), or apply the stage update of
+// CCFVM/main.F90:92-101 in place (op 1; no other cell reads this cell's
+// state during a stage).  rev: the XCDs walk their slices of blocks from the
+// far end.  SL: the block's records are first copied to LDS, so the
+// neighbours inside the block (most of them, the cells being
+// Hilbert-ordered) are read from there instead of through L2.
+template <typename R, int FLUX, bool SL>
+__global__ __launch_bounds__(BLK) void k_stage(DevT<R> d, Gas<R> gr, int op, int rev, double ak,
+                                               double bk, int write_res) {
+  extern __shared__ double lds_raw[];
+  R* srec = reinterpret_cast<R*>(lds_raw);  // [BLK][RW] when SL
+  const int base = xcd_block_dir(blockIdx.x, gridDim.x, rev != 0) * BLK;
+  const int c = base + threadIdx.x;
+  if (SL) {
+    stage_block_recs(d, srec, base, min(BLK, d.noc - base));
+    __syncthreads();
+  }
+  if (c >= d.noc || d.err[0]) return;
+  double r[4];
+  const int ekey = gather_residual<R, FLUX, SL>(d, srec, base, c, gr, r);
+  if (ekey != INT_MAX) set_err(d, DERR_ROE, ekey);
+  stage_end<R>(d, c, op, ak, bk, write_res, r);
+}
+
+// ---- whole inviscid RK3 iterations
+// The reference refreshes the primitives, gradients and limiter values once
+// per iteration (CCFVM/main.F90:59-86) and never inside the stage loop
+// (:88-109), so the interior fluxes of the three stages are evaluated from
+// the same inputs and are the same numbers; of a residual only the wall
+// faces, whose ghost mirrors the inner cell's current state
+// (CCFVM/boundCond.F90), change from stage to stage.  A whole iteration
+// therefore evaluates the interior residual once.  For a cell without
+// boundary faces the three stage updates are then a chain in its registers
+// (k_rk3, k_rk3_blk): the state is read and written once per iteration.  The
+// cells with boundary faces (k_rk3_bcell; a few thousand of two million) keep
+// their interior fluxes and evaluate their wall faces in every stage.  The same sums in the same order as the
+// routine-by-routine stages.
+template <typename R>
+__device__ __forceinline__ void rk3_step(int stage, const double* q0, double dta, const double* r,
+                                         double* q) {
+  const double ak = stage == 0 ? 0.0 : stage == 1 ? 3.0 / 4.0 : 1.0 / 3.0;
+  const double bk = stage == 0 ? 1.0 : stage == 1 ? 1.0 / 4.0 : 2.0 / 3.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q[i] = rk_update1(ak, q0[i], bk, q[i], dta, r[i]);
+}
+
+// The three updates of an interior cell c with residual r; returns its new
+// state and its squared residual.
+template <typename R>
+__device__ __forceinline__ double rk3_cell(const DevT<R>& d, int c, const double* r, int write_res,
+                                           double* q) {
+  double dta = ld_nt(d.dta + c), q0[4];
+  ld4d_nt(d.qc + (size_t)c * 4, q0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q[i] = q0[i];
+#pragma unroll
+  for (int st = 0; st < 3; ++st) rk3_step<R>(st, q0, dta, r, q);
+  st4d_nt(d.qc + (size_t)c * 4, q);
+  if (write_res) st4d_nt(d.res + (size_t)c * 4, r);
+  double sq = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sq = sq + r[i] * r[i];
+  return sq;
+}
+
+// Place of cell c of block b in the list of the cells with boundary faces
+// (ascending: a few steps through the block's own part of it).
+template <typename R>
+__device__ __forceinline__ int bc_index(const DevT<R>& d, int b, int c) {
+  int t = d.bc_ptr[b];
+  while (t < d.nbc - 1 && d.bc_cell[t] != c) ++t;
+  return t;
+}
+
+template <typename R, int FLUX, bool SL>
+__device__ __forceinline__ void rk3_body(const DevT<R>& d, VBlock vb, const Gas<R>& gr,
+                                         const Gas<double>& g, int rev, int write_res, int epi) {
+  extern __shared__ double lds_raw[];
+  R* srec = reinterpret_cast<R*>(lds_raw);  // [BLK][RW] when SL
+  const int base = xcd_block_dir(vb.b, vb.n, rev != 0) * BLK;
+  const int c = base + threadIdx.x;
+  if (SL) {
+    stage_block_recs(d, srec, base, min(BLK, d.noc - base));
+    __syncthreads();
+  }
+  double sq = 0.0, q[4] = {0.0, 0.0, 0.0, 0.0};
+  const int info = c < d.noc && !d.err[0] ? d.cnf[c] : -1;
+  const bool have = info >= 0 && (info >> 8) == 0;
+  // the cells with boundary faces: their interior fluxes for k_rk3_bcell in
+  // the mixed form (FP64: that kernel evaluates them)
+  if (sizeof(R) == 4 ? info >= 0 : have) {
+    double r[4];
+    R* keep = sizeof(R) == 4 && !have ? d.bcF + (size_t)bc_index(d, base / BLK, c) * 4 : nullptr;
+    const int ekey =
+        gather_residual<R, FLUX, SL, false>(d, srec, base, c, gr, r, keep, 4 * (size_t)d.nbc);
+    if (ekey != INT_MAX) set_err(d, DERR_ROE, ekey);
+    if (have) sq = rk3_cell<R>(d, c, r, write_res, q);
+  }
+  rk3_finish<R, false>(d, vb.b, g, c, have, q, sq, epi);
+}
+template <typename R, int FLUX, bool SL>
+__global__ __launch_bounds__(BLK) void k_rk3(DevT<R> d, Gas<R> gr, Gas<double> g, int rev,
+                                             int write_res, int epi) {
+  rk3_body<R, FLUX, SL>(d, hw_block(), gr, g, rev, write_res, epi);
+}
+
+// The cells with boundary faces, BC_CELLS to a block, after the block's other
+// cells.  stored: their interior fluxes were left in bcF by the pass over the
+// other cells (the block-shared form, and the mixed form: an FP32 flux
+// evaluated here could round differently than in a routine's residual), else
+// they are evaluated here.  The kernel is a chain of latencies (a few dozen blocks), so
+// its work is spread over the lanes, its lists are packed (bc_tab: one load
+// where cnf, sl_nbr, sl_face and fbc would be a chain of three) and its code
+// kept short: one wave per face slot
+// evaluates that slot's fluxes, the first wave sums them and applies the
+// stage updates, one lane per cell.  Interior and farfield fluxes do not
+// change over the stages; a wall's is evaluated in each.  slot0: the blocks'
+// first slot among the partials.  A wall face failing in a later stage counts
+// after every failure of the earlier ones (the key gets the stage in front,
+// see set_err).
+constexpr int BC_CELLS = BLK / MAXF;
+template <typename R, int FLUX>
+__device__ __forceinline__ void rk3_bcell_body(const DevT<R>& d, VBlock vb, int slot0,
+                                               const Gas<R>& gr, const BndOpts& bo, int stored,
+                                               int write_res, int epi) {
+  static_assert(BC_CELLS == 64, "one wave per face slot");
+  constexpr int RW = Layout<R>::RW, FW = Layout<R>::FW;
+  __shared__ double s_F[MAXF][4][BC_CELLS];
+  __shared__ double s_q[4][BC_CELLS];
+  __shared__ int s_in[MAXF][BC_CELLS];  // the cell is the slot's face's `in`
+  const int l = threadIdx.x % BC_CELLS, s = threadIdx.x / BC_CELLS;
+  const int t = vb.b * BC_CELLS + l;
+  const bool run = t < d.nbc && !d.err[0];
+  const int tc = min(t, d.nbc - 1), c = d.bc_cell[tc];
+  const int4 tab = d.bc_tab[(size_t)s * d.nbc + tc];
+  const int nf = tab.w & 0xff, ni = nf - (tab.w >> 8), f = tab.y;
+  R own[RW];
+  int k = -1;  // this slot's boundary face
+  if (run && s < ni) {
+    const bool in_side = tab.x >= 0;
+    const int n = in_side ? tab.x : ~tab.x;
+    R fx[4];
+    if (sizeof(R) == 4 || stored) {
+      ldv<R, 4>(d.bcF + ((size_t)s * d.nbc + tc) * 4, fx);
+    } else {
+      R ra[RW], rb[RW], fr[FW];
+      face_rec(d, f, fr);
+      ldv<R, RW>(d.rec + (size_t)(in_side ? c : n) * RW, ra);
+      ldv<R, RW>(d.rec + (size_t)(in_side ? n : c) * RW, rb);
+      if (!face_flux_ab<R, FLUX>(gr, ra, rb, fr, fx)) set_err(d, DERR_ROE, d.nbf + d.fref[f]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_F[s][i][l] = (double)fx[i];
+    s_in[s][l] = in_side;
+  } else if (run && s < nf) {
+    ldv<R, RW>(d.rec + (size_t)c * RW, own);
+    k = tab.x - d.noc;
+  }
+  const bool have = run && s == 0;
+  double sq = 0.0, q[4] = {0.0, 0.0, 0.0, 0.0}, q0[4] = {0.0, 0.0, 0.0, 0.0}, r[4], dta = 0.0;
+  if (have) {
+    dta = d.dta[c];
+    ld4d(d.qc + (size_t)c * 4, q0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_q[i][l] = q[i] = q0[i];
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int st = 0; st < 3; ++st) {
+    if (k >= 0 && (st == 0 || tab.z == WALL)) {
+      double F[4];
+      if (!bface_one<R, FLUX>(d, bo, tab.z, k, f, own, [&](int i) { return s_q[i][l]; }, F))
+        set_err(d, DERR_ROE, st * (d.nbf + d.nof) + k);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s_F[s][i][l] = F[i];
+    }
+    __syncthreads();
+    if (have) {
+      // the boundary fluxes first, as the reference's loops add them
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = 0.0;
+#pragma unroll 1
+      for (int j = ni; j < nf; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = r[i] + s_F[j][i][l];
+#pragma unroll 1
+      for (int j = 0; j < ni; ++j) {
+        const bool in_side = s_in[j][l];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = in_side ? r[i] + s_F[j][i][l] : r[i] - s_F[j][i][l];
+      }
+      const double ak = st == 0 ? 0.0 : st == 1 ? 3.0 / 4.0 : 1.0 / 3.0;
+      const double bk = st == 0 ? 1.0 : st == 1 ? 1.0 / 4.0 : 2.0 / 3.0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s_q[i][l] = q[i] = rk_update1(ak, q0[i], bk, q[i], dta, r[i]);
+    }
+    __syncthreads();
+  }
+  if (have) {
+    st4d(d.qc + (size_t)c * 4, q);
+    if (write_res) st4d(d.res + (size_t)c * 4, r);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sq = sq + r[i] * r[i];
+  }
+  rk3_finish<R, true>(d, slot0 + vb.b, bo.g, c, have, q, sq, epi);
+}
+template <typename R, int FLUX>
+__global__ __launch_bounds__(BLK) void k_rk3_bcell(DevT<R> d, int slot0, Gas<R> gr, BndOpts bo,
+                                                   int stored, int write_res, int epi) {
+  rk3_bcell_body<R, FLUX>(d, hw_block(), slot0, gr, bo, stored, write_res, epi);
+}
+
+// The interior fluxes of a block's cells, each evaluated once per block
+// instead of once per adjacent cell.  Phase 1: the block's threads walk the
+// interior faces touched by its BLK cells (Hilbert-ordered, so about 1.65
+// faces per cell instead of 3), evaluate each flux once and keep it in LDS.
+// Phase 2 (blk_residual): each cell sums its interior fluxes from LDS in its
+// slot order (the reference's accumulation order).  SL as in k_stage.
 // LDS: [BLK][RW] records when SL, then [bf_max][4] fluxes; when SL and the
 // list has at most 2 BLK faces, the fluxes are held in registers until every
 // thread is done with the records and then written over them, so the block
-// needs no more LDS than its records.
+// needs no more LDS than its records.  Returns the flux list; *run: no error
+// was pending when the block started (uniform over the block).
 template <typename R, int FLUX, bool SL>
-__device__ __forceinline__ void stage_blk_body(const DevT<R>& d, VBlock vb, Gas<R> gr, int mode,
-                                               double ak, double bk, int write_res,
-                                               const Gas<double>& g, int epi) {
-  const int op = mode & 3, src = (mode >> 2) & 3;
-  const bool rev = (mode & 16) != 0;
+__device__ __forceinline__ const R* blk_fluxes(const DevT<R>& d, int b, const Gas<R>& gr,
+                                               bool* run) {
   constexpr int RW = Layout<R>::RW, FW = Layout<R>::FW;
   extern __shared__ double lds_raw[];
   R* srec = reinterpret_cast<R*>(lds_raw);
   R* fl = srec + (SL ? BLK * RW : 0);
-  __shared__ double sh[1][BLK];
   __shared__ int s_err;
   if (threadIdx.x == 0) s_err = d.err[0];
-  const int b = xcd_block_dir(vb.b, vb.n, rev), base = b * BLK;
+  const int base = b * BLK;
   if (SL) stage_block_recs(d, srec, base, min(BLK, d.noc - base));
   __syncthreads();
-  const bool run = s_err == 0;  // uniform over the block
-  const int j0 = d.bf_ptr[b], nj = run ? d.bf_ptr[b + 1] - j0 : 0;
+  *run = s_err == 0;
+  const int j0 = d.bf_ptr[b], nj = *run ? d.bf_ptr[b + 1] - j0 : 0;
   if (SL && d.bf_max <= 2 * BLK) {
     R F2[2][4];
 #pragma unroll
@@ -1074,66 +1237,88 @@ __device__ __forceinline__ void stage_blk_body(const DevT<R>& d, VBlock vb, Gas<
     for (int i = 0; i < 4; ++i) fl[j * 4 + i] = F[i];
   }
   __syncthreads();
-  const int c = base + threadIdx.x;
+  return fl;
+}
+
+// The sum of cell c's boundary fluxes (BND) and interior fluxes.
+template <typename R, bool BND>
+__device__ __forceinline__ void blk_residual(const DevT<R>& d, int c, int info, const R* fl,
+                                             double* r) {
+  const int noc = d.noc, nf = info & 0xff, nb = BND ? info >> 8 : 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = 0.0;
+  for (int s = nf - nb; BND && s < nf; ++s) {
+    int k = ld_nt(d.sl_nbr + s * noc + c) - noc;
+    double F[4];
+    ld4d(d.bres + (size_t)k * 4, F);
+    for (int i = 0; i < 4; ++i) r[i] = r[i] + F[i];
+  }
+  int sl[MAXF];
+#pragma unroll
+  for (int s = 0; s < MAXF; ++s)
+    if (s < nf - nb) sl[s] = ld_nt(d.sl_loc + s * noc + c);
+#pragma unroll
+  for (int s = 0; s < MAXF; ++s) {
+    if (s >= nf - nb) break;
+    int l = sl[s];
+    bool in_side = l >= 0;
+    l = in_side ? l : ~l;
+    if (in_side) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = r[i] + (double)fl[l * 4 + i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = r[i] - (double)fl[l * 4 + i];
+    }
+  }
+}
+
+// k_stage with the block's fluxes evaluated once.
+template <typename R, int FLUX, bool SL>
+__global__ __launch_bounds__(BLK) void k_stage_blk(DevT<R> d, Gas<R> gr, int op, int rev,
+                                                   double ak, double bk, int write_res) {
+  const int b = xcd_block_dir(blockIdx.x, gridDim.x, rev != 0);
+  bool run;
+  const R* fl = blk_fluxes<R, FLUX, SL>(d, b, gr, &run);
+  const int c = b * BLK + threadIdx.x;
+  if (!run || c >= d.noc) return;
+  double r[4];
+  blk_residual<R, true>(d, c, ld_nt(d.cnf + c), fl, r);
+  stage_end<R>(d, c, op, ak, bk, write_res, r);
+}
+
+// k_rk3 with the block's fluxes evaluated once.
+template <typename R, int FLUX, bool SL>
+__device__ __forceinline__ void rk3_blk_body(const DevT<R>& d, VBlock vb, const Gas<R>& gr,
+                                             const Gas<double>& g, int rev, int write_res,
+                                             int epi) {
+  const int b = xcd_block_dir(vb.b, vb.n, rev != 0);
+  bool run;
+  const R* fl = blk_fluxes<R, FLUX, SL>(d, b, gr, &run);
+  const int c = b * BLK + threadIdx.x;
   double sq = 0.0, q[4] = {0.0, 0.0, 0.0, 0.0};
-  bool have = false;
-  if (run && c < d.noc) {
-    const int noc = d.noc;
-    int info = ld_nt(d.cnf + c), nf = info & 0xff, nb = info >> 8;
-    double r[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int s = nf - nb; s < nf; ++s) {
-      int k = ld_nt(d.sl_nbr + s * noc + c) - noc;
-      double F[4];
-      ld4d(d.bres + (size_t)k * 4, F);
-      for (int i = 0; i < 4; ++i) r[i] = r[i] + F[i];
+  const int info = run && c < d.noc ? ld_nt(d.cnf + c) : -1;
+  const bool have = info >= 0 && (info >> 8) == 0;
+  if (info >= 0 && !have) {
+    // a cell with boundary faces: its interior fluxes for k_rk3_bcell
+    const int t = bc_index(d, b, c);
+    const int ni = (info & 0xff) - (info >> 8);
+    for (int s = 0; s < ni; ++s) {
+      const int sl = d.sl_loc[s * d.noc + c], j = sl >= 0 ? sl : ~sl;
+      stv<R, 4>(d.bcF + ((size_t)s * d.nbc + t) * 4, fl + j * 4);
     }
-    int sl[MAXF];
-#pragma unroll
-    for (int s = 0; s < MAXF; ++s)
-      if (s < nf - nb) sl[s] = ld_nt(d.sl_loc + s * noc + c);
-#pragma unroll
-    for (int s = 0; s < MAXF; ++s) {
-      if (s >= nf - nb) break;
-      int l = sl[s];
-      bool in_side = l >= 0;
-      l = in_side ? l : ~l;
-      if (in_side) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = r[i] + (double)fl[l * 4 + i];
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = r[i] - (double)fl[l * 4 + i];
-      }
-    }
-    if (op == 0 || write_res) st4d_nt(d.res + (size_t)c * 4, r);
-    if (op >= 1) {
-      double dta = ld_nt(d.dta + c), o[4];
-      ld4d_nt(stage_old(d, src) + (size_t)c * 4, o);
-      if (src == 1) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) q[i] = o[i];
-      } else {
-        ld4d_nt(stage_in(d, src) + (size_t)c * 4, q);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) q[i] = rk_update1(ak, o[i], bk, q[i], dta, r[i]);
-      st4d_nt(stage_out(d, src) + (size_t)c * 4, q);
-      have = true;
-    }
-    if (op == 2)
-      for (int i = 0; i < 4; ++i) sq = sq + r[i] * r[i];
   }
-  if (op == 2) {
-    block_reduce<1>(sh, &sq, OpAdd());
-    if (threadIdx.x == 0) d.part[vb.b] = sq;
+  if (have) {
+    double r[4];
+    blk_residual<R, false>(d, c, info, fl, r);
+    sq = rk3_cell<R>(d, c, r, write_res, q);
   }
-  if (epi) prim_epilogue<R>(d, vb, g, c, have, q);
+  rk3_finish<R, false>(d, vb.b, g, c, have, q, sq, epi);
 }
 template <typename R, int FLUX, bool SL>
-__global__ __launch_bounds__(BLK) void k_stage_blk(DevT<R> d, Gas<R> gr, int mode, double ak,
-                                                   double bk, int write_res, Gas<double> g,
-                                                   int epi) {
-  stage_blk_body<R, FLUX, SL>(d, hw_block(), gr, mode, ak, bk, write_res, g, epi);
+__global__ __launch_bounds__(BLK) void k_rk3_blk(DevT<R> d, Gas<R> gr, Gas<double> g, int rev,
+                                                 int write_res, int epi) {
+  rk3_blk_body<R, FLUX, SL>(d, hw_block(), gr, g, rev, write_res, epi);
 }
 
 // Sutherland viscosity of the interior cells from the current state,

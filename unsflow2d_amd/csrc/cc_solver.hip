@@ -86,9 +86,10 @@ struct ufx_cc {
   size_t stage_lds = 0;          // LDS bytes per block of the stage kernel
   size_t lds_list = 0, lds_recs = 0;  // LDS of the block flux list / records
   bool lds_overlay = false;            // the flux list fits over the records (at most 2 BLK faces)
-  // alternate traversal: in RK stages 1 and 3 the XCDs walk their slices of
-  // blocks from the far end, so each stage starts on the data the pass
-  // before it touched last, which the 256 MB memory-side cache still holds
+  // alternate traversal: in the residual pass of a whole iteration and in
+  // the routines' RK stages 1 and 3 the XCDs walk their slices of blocks
+  // from the far end, so the pass starts on the data the pass before it
+  // touched last, which the 256 MB memory-side cache still holds
   // (UFX_SERPENTINE=0: all passes forward)
   int stage_rev = 10;                  // bit s: stage s walks its blocks from the far end
   hipStream_t stream = nullptr;
@@ -105,6 +106,7 @@ struct ufx_cc {
   unsigned prof_mask = ~0u;        // kernel categories timed while profiling
   double* d_out = nullptr;         // small device results (residual norms)
   int nblk_cell = 0, nblk_all = 0, nblk_pt = 0, nblk_face = 0;
+  int nblk_bc = 0;               // blocks of the cells with boundary faces
   double* d_hist = nullptr;
   int hist_cap = 0;
   double* cirs_tmp = nullptr;    // [noc][4] the first smoothing sweep's result
@@ -258,9 +260,10 @@ void decode_error(const ufx_cc* x, const int* e, int* kind, int* face, int* cell
   *kind = e[0];
   *face = 0;
   *cell = 0;
-  if (e[0] == DERR_ROE && e[3] >= 0 && e[3] < x->nbf + x->nfi) {
+  const int key = e[3] >= 0 ? e[3] % std::max(1, x->nbf + x->nof) : -1;  // without the stage
+  if (e[0] == DERR_ROE && key >= 0 && key < x->nbf + x->nfi) {
     // boundary faces are keyed by their ordinal, interior ones after them
-    int f = e[3] < x->nbf ? x->nfi + e[3] : e[3] - x->nbf;
+    int f = key < x->nbf ? x->nfi + key : key - x->nbf;
     *face = f + 1;
     *cell = x->fin_ref[f] + 1;
   } else if (e[0] == DERR_AREA && e[3] >= 0 && e[3] < x->nof) {
@@ -428,29 +431,30 @@ int restore_dtla(ufx_cc* x, DevT<R>& d) {
   return launch_check();
 }
 
+// The residual routine by routine: the boundary faces, then the interior
+// residual of every cell, stored (op 0) or with the stage update (op 1).
 template <typename R>
-int run_stage_kernel(ufx_cc* x, DevT<R>& d, int mode, double ak, double bk, int write_res,
-                     int epi = 0) {
-  const int src = (mode >> 2) & 3;
+int run_stage_kernel(ufx_cc* x, DevT<R>& d, int op, int rev, double ak, double bk,
+                     int write_res) {
   int visc = x->p.flow != UFX_FLOW_INVISCID;
   const Gas<R>& gr = gas_of<R>(x);
   int nbb = nblocks(x->nbf);
 #define KS(F)                                                                                   \
   do {                                                                                          \
     if (x->nbf > 0)                                                                             \
-      LAUNCH(x, UFX_K_BFACE, (k_bface<R, F>), nbb, d, x->g, visc, x->p.iwall, x->p.t_wall, src); \
+      LAUNCH(x, UFX_K_BFACE, (k_bface<R, F>), nbb, d, x->g, visc, x->p.iwall, x->p.t_wall);     \
     if (x->stage_shared && x->stage_local)                                                      \
       LAUNCH_LDS(x, UFX_K_STAGE, (k_stage_blk<R, F, true>), x->nblk_cell, x->stage_lds, d, gr,  \
-                 mode, ak, bk, write_res, x->g, epi);                                           \
+                 op, rev, ak, bk, write_res);                                                   \
     else if (x->stage_shared)                                                                   \
       LAUNCH_LDS(x, UFX_K_STAGE, (k_stage_blk<R, F, false>), x->nblk_cell, x->stage_lds, d, gr, \
-                 mode, ak, bk, write_res, x->g, epi);                                           \
+                 op, rev, ak, bk, write_res);                                                   \
     else if (x->stage_local)                                                                    \
-      LAUNCH_LDS(x, UFX_K_STAGE, (k_stage<R, F, true>), x->nblk_cell, x->stage_lds, d, gr,      \
-                 mode, ak, bk, write_res, x->g, epi);                                           \
+      LAUNCH_LDS(x, UFX_K_STAGE, (k_stage<R, F, true>), x->nblk_cell, x->stage_lds, d, gr, op,  \
+                 rev, ak, bk, write_res);                                                       \
     else                                                                                        \
-      LAUNCH(x, UFX_K_STAGE, (k_stage<R, F, false>), x->nblk_cell, d, gr, mode, ak, bk,         \
-             write_res, x->g, epi);                                                             \
+      LAUNCH(x, UFX_K_STAGE, (k_stage<R, F, false>), x->nblk_cell, d, gr, op, rev, ak, bk,      \
+             write_res);                                                                        \
   } while (0)
   switch (x->p.flux) {
     case UFX_FLUX_ROE: KS(1); break;
@@ -459,6 +463,42 @@ int run_stage_kernel(ufx_cc* x, DevT<R>& d, int mode, double ak, double bk, int 
     default: KS(4); break;
   }
 #undef KS
+  return launch_check();
+}
+
+// The three stages of a whole inviscid RK3 iteration (k_rk3 and
+// k_rk3_bcell): the cells without boundary faces, then those with.  epi: also
+// the next iteration's primitives.
+template <typename R>
+int run_rk3(ufx_cc* x, DevT<R>& d, int write_res, int epi) {
+  const Gas<R>& gr = gas_of<R>(x);
+  const int rev = (x->stage_rev >> 1) & 1;
+  const BndOpts bo{x->g, 0, x->p.iwall, x->p.t_wall};
+#define KR(F)                                                                                   \
+  do {                                                                                          \
+    if (x->stage_shared && x->stage_local)                                                      \
+      LAUNCH_LDS(x, UFX_K_STAGE, (k_rk3_blk<R, F, true>), x->nblk_cell, x->stage_lds, d, gr,    \
+                 x->g, rev, write_res, epi);                                                    \
+    else if (x->stage_shared)                                                                   \
+      LAUNCH_LDS(x, UFX_K_STAGE, (k_rk3_blk<R, F, false>), x->nblk_cell, x->stage_lds, d, gr,   \
+                 x->g, rev, write_res, epi);                                                    \
+    else if (x->stage_local)                                                                    \
+      LAUNCH_LDS(x, UFX_K_STAGE, (k_rk3<R, F, true>), x->nblk_cell, x->stage_lds, d, gr, x->g,  \
+                 rev, write_res, epi);                                                          \
+    else                                                                                        \
+      LAUNCH(x, UFX_K_STAGE, (k_rk3<R, F, false>), x->nblk_cell, d, gr, x->g, rev, write_res,   \
+             epi);                                                                              \
+    if (x->nblk_bc > 0)                                                                         \
+      LAUNCH(x, UFX_K_BFACE, (k_rk3_bcell<R, F>), x->nblk_bc, d, x->nblk_cell, gr, bo,          \
+             x->stage_shared ? 1 : 0, write_res, epi);                                          \
+  } while (0)
+  switch (x->p.flux) {
+    case UFX_FLUX_ROE: KR(1); break;
+    case UFX_FLUX_AUSM: KR(2); break;
+    case UFX_FLUX_VANLEER: KR(3); break;
+    default: KR(4); break;
+  }
+#undef KR
   return launch_check();
 }
 
@@ -487,7 +527,7 @@ int run_cirs(ufx_cc* x, DevT<R>& d, bool upd = false, double ak = 0.0, double bk
 template <typename R>
 int run_residual_full(ufx_cc* x, DevT<R>& d, bool upd = false, double ak = 0.0, double bk = 0.0,
                       bool* upd_done = nullptr) {
-  if (int rc = run_stage_kernel(x, d, 0, 0.0, 0.0, 1)) return rc;
+  if (int rc = run_stage_kernel(x, d, 0, 0, 0.0, 0.0, 1)) return rc;
   if (x->p.flow != UFX_FLOW_INVISCID) {
     if (x->p.grad != UFX_GRAD_GGFC) {
       if (int rc = run_ggfc_face(x, d)) return rc;
@@ -519,17 +559,12 @@ const double RK_B[3] = {1.0, 1.0 / 4.0, 2.0 / 3.0};
 
 // One Runge-Kutta stage: residual and update fused in one pass when nothing
 // else contributes to the residual, else the full residual then the update.
-// whole: a stage of a whole iteration (its states in qc and qs, see
-// stage_old/in/out), else routine by routine (qold and qc); epi: the stage
-// also refreshes the next iteration's primitives (prim_epilogue).
+// norm: also the partials of the residual norm (whole iterations).
 template <typename R>
-int run_stage(ufx_cc* x, DevT<R>& d, int stage, bool norm, bool write_res, bool whole,
-              bool epi = false) {
+int run_stage(ufx_cc* x, DevT<R>& d, int stage, bool norm) {
   double ak = RK_A[stage - 1], bk = RK_B[stage - 1];
   if (x->p.flow == UFX_FLOW_INVISCID && !x->p.irs)
-    return run_stage_kernel(x, d, (norm ? 2 : 1) | ((whole ? stage : 0) << 2) |
-                                      ((x->stage_rev >> stage) & 1 ? 16 : 0),
-                            ak, bk, write_res ? 1 : 0, epi ? 1 : 0);
+    return run_stage_kernel(x, d, 1, (x->stage_rev >> stage) & 1, ak, bk, 1);
   bool updated = false;
   if (int rc = run_residual_full(x, d, true, ak, bk, &updated)) return rc;
   if (!updated)
@@ -592,7 +627,7 @@ int run_iteration(ufx_cc* x, DevT<R>& d, int iter, int k) {
   bool visc = x->p.flow != UFX_FLOW_INVISCID;
   // prim refresh, qold (save_old commutes with avg_c2v and the time step),
   // positivity and the global range (re-armed by the previous norm)
-  // the fused RK3 stages keep the start state in qc (no qold copy)
+  // the fused RK3 stages read the start state from qc (no qold copy)
   const bool fused = x->p.timemode == UFX_TIME_RK3 && !visc && !x->p.irs;
   // the last stage of a fused iteration refreshes the next iteration's
   // primitives itself (not with the diamond-path gradient, whose face pass
@@ -604,20 +639,24 @@ int run_iteration(ufx_cc* x, DevT<R>& d, int iter, int k) {
   if (refresh)
     if (int rc = run_prim(x, d, 1, fused ? 2 : 1, lim ? 1 : 0)) return rc;
   // vertex averages, with the range reduction as one more block
-  if (int rc = lim ? run_avg_range(x, d, refresh ? x->nblk_all : x->nblk_cell) : run_avg(x, d))
+  if (int rc = lim ? run_avg_range(x, d, refresh ? x->nblk_all : x->nblk_cell + x->nblk_bc)
+                   : run_avg(x, d))
     return rc;
   // gradient, limiter and time step in one pass over the cells; the
   // temperature gradient only when the viscous flux needs it
   if (int rc = run_gradient(x, d, visc, lim, true, x->cfl, fused ? 0 : 1)) return rc;
-  if (x->p.timemode == UFX_TIME_RK3) {
+  int nparts = x->nblk_cell;  // block partials of the norm
+  if (fused) {
+    if (int rc = run_rk3(x, d, x->keep_res ? 1 : 0, epi ? 1 : 0)) return rc;
+    nparts += x->nblk_bc;
+  } else if (x->p.timemode == UFX_TIME_RK3) {
     for (int s = 1; s <= 3; ++s)
-      if (int rc = run_stage(x, d, s, s == 3, s == 3 && x->keep_res, fused, s == 3 && epi))
-        return rc;
+      if (int rc = run_stage(x, d, s, s == 3)) return rc;
   } else {
     if (int rc = run_lusgs(x, d)) return rc;
     LAUNCH(x, UFX_K_NORM, k_sumsq<R>, x->nblk_cell, d);
   }
-  LAUNCH(x, UFX_K_NORM, k_norm_final<R>, 1, d, x->nblk_cell, iter == 1, x->d_hist, k);
+  LAUNCH(x, UFX_K_NORM, k_norm_final<R>, 1, d, nparts, iter == 1, x->d_hist, k);
   x->prims_next = epi;
   return launch_check();
 }
@@ -908,6 +947,29 @@ int build_dev(ufx_cc* x, DevT<R>& d, const Mesh& m, const std::vector<int>& sl_f
     d.fpt = p;
   }
   UP(fbc, fbc); UP(bface, bface); UP(bcell, bcell);
+  {
+    std::vector<int> bc_cell, bc_ptr;
+    for (int s = 0; s < noc; ++s) {
+      if (s % BLK == 0) bc_ptr.push_back((int)bc_cell.size());
+      if (cnf[s] >> 8) bc_cell.push_back(s);
+    }
+    d.nbc = (int)bc_cell.size();
+    x->nblk_bc = (d.nbc + BC_CELLS - 1) / BC_CELLS;
+    UP(bc_cell, bc_cell);
+    std::vector<int4> bc_tab((size_t)MAXF * d.nbc, make_int4(0, 0, 0, 0));
+    for (int t = 0; t < d.nbc; ++t) {
+      const int c = bc_cell[t], nf = cnf[c] & 0xff, ni = nf - (cnf[c] >> 8);
+      for (int s = 0; s < MAXF; ++s) {
+        const size_t q = (size_t)s * noc + c;
+        const int nb = s < nf ? sl_nbr[q] : 0;
+        bc_tab[(size_t)s * d.nbc + t] =
+            make_int4(nb, s < nf ? sl_face[q] : 0, s >= ni && s < nf ? fbc[nb - noc] : 0, cnf[c]);
+      }
+    }
+    UP(bc_tab, bc_tab);
+    UP(bc_ptr, bc_ptr);
+    AL(bcF, 4 * (size_t)MAXF * d.nbc);
+  }
   UP(sl_face, sl_face); UP(sl_nbr, sl_nbr); UP(cnf, cnf);
   UP(bf_ptr, sl.bf_ptr); UP(sl_loc, sl.sl_loc);
   d.bf_max = sl.bf_max;
@@ -939,12 +1001,13 @@ int build_dev(ufx_cc* x, DevT<R>& d, const Mesh& m, const std::vector<int>& sl_f
     std::vector<R> qpc((size_t)noc * 4, R(0));
     UP(qpc, qpc);
   }
-  AL(fw, nof); AL(qT, ncell); AL(qTc, noc); AL(gT, 2 * (size_t)noc); AL(qold, 4 * (size_t)noc); AL(qs, 4 * (size_t)noc);
+  AL(fw, nof); AL(qT, ncell); AL(qTc, noc); AL(gT, 2 * (size_t)noc); AL(qold, 4 * (size_t)noc);
   AL(res, 4 * (size_t)noc); AL(dt, noc); AL(dta, noc); AL(la, noc); AL(fla, nof); AL(fmu, nof);
   if (x->p.flow != UFX_FLOW_INVISCID) AL(fvis, 4 * (size_t)nof);
   AL(cmul, ncell); AL(prec, (size_t)nop * PW); AL(fgrad, (size_t)nof * 10);
   AL(bflux, 2 * (size_t)std::max(1, nbf)); AL(bres, 4 * (size_t)std::max(1, nbf));
-  AL(part, (size_t)std::max(x->nblk_all, 1) * 8); AL(rpart, (size_t)std::max(x->nblk_all, 1) * 8);
+  const size_t nparts = (size_t)std::max(x->nblk_all, x->nblk_cell + x->nblk_bc);
+  AL(part, nparts); AL(rpart, nparts * 8);
   AL(scal, SC_NSCAL); AL(range, 8); AL(err, 4); AL(lower, 4 * (size_t)noc); AL(upper, 4 * (size_t)noc);
 #undef UP
 #undef AL
@@ -1334,7 +1397,7 @@ int ufx_cc_rk_stage(ufx_cc* x, int stage) {
   if (int rc = check_routine(x)) return rc;
   if (stage < 1 || stage > 3) { set_error("stage must be 1..3"); return UFX_ERR_ARG; }
   if (int rc = check_qold(x, "ufx_cc_rk_stage")) return rc;
-  return with_dev(x, [&](auto& d) { return run_stage(x, d, stage, false, true, false); });
+  return with_dev(x, [&](auto& d) { return run_stage(x, d, stage, false); });
 }
 
 int ufx_cc_lusgs(ufx_cc* x) {
@@ -1762,7 +1825,7 @@ struct ufx_cc_batch {
 namespace {
 
 // block tables: all cells (incl. ghosts), vertices, faces, interior cells,
-// boundary faces, one block per case
+// cells with boundary faces, one block per case
 enum { T_ALL, T_PT, T_FACE, T_CELL, T_BF, T_CASE, T_N };
 
 template <typename R> DevT<R>& dev_of(ufx_cc* x);
@@ -1797,7 +1860,7 @@ int batch_write(ufx_cc_batch* b) {
     e.nblk_pt = x->nblk_pt;
     e.nblk_face = x->nblk_face;
     e.nblk_cell = x->nblk_cell;
-    e.nblk_bf = x->nbf > 0 ? nblocks(x->nbf) : 0;
+    e.nblk_bc = x->nblk_bc;
     b->hist_seen[i] = x->d_hist;
     ids.push_back(i);
   }
@@ -1806,7 +1869,7 @@ int batch_write(ufx_cc_batch* b) {
     for (int i : ids) {
       const CaseDesc<R>& e = desc[i];
       const int nb = t == T_ALL ? e.nblk_all : t == T_PT ? e.nblk_pt : t == T_FACE ? e.nblk_face
-                   : t == T_CELL ? e.nblk_cell : t == T_BF ? e.nblk_bf : 1;
+                   : t == T_CELL ? e.nblk_cell : t == T_BF ? e.nblk_bc : 1;
       for (int k = 0; k < nb; ++k) map.push_back(make_int4(i, k, nb, 0));
     }
     b->cnt[t] = map.size() - b->off[t];
@@ -1858,34 +1921,28 @@ int batch_iteration(ufx_cc_batch* b, ufx_cc* x0, int k, double cfl, int keep, bo
   if (x0->p.grad == UFX_GRAD_GG) KMC(G_GG);
   else KMC(G_LSQR);
 #undef KMC
-  for (int st = 1; st <= 3; ++st) {
-    const double ak = RK_A[st - 1], bk = RK_B[st - 1];
-    const int mode = (st == 3 ? 2 : 1) | (st << 2) | ((x0->stage_rev >> st) & 1 ? 16 : 0),
-              wr = st == 3 && keep ? 1 : 0;
-    const int epi = st == 3 ? 1 : 0;
-    const size_t lds = b->stage_lds;
+  const int rev = (x0->stage_rev >> 1) & 1;
+  const size_t lds = b->stage_lds;
 #define KMS(F)                                                                                  \
   do {                                                                                          \
-    if (b->cnt[T_BF]) km_bface<R, F><<<G(T_BF), BLK, 0, s>>>(cs, M(T_BF), 0, st);               \
     if (x0->stage_shared && x0->stage_local)                                                    \
-      km_stage_blk<R, F, true><<<G(T_CELL), BLK, lds, s>>>(cs, M(T_CELL), mode, ak, bk, wr,     \
-                                                           epi);                                \
+      km_rk3_blk<R, F, true><<<G(T_CELL), BLK, lds, s>>>(cs, M(T_CELL), rev, keep, 1);          \
     else if (x0->stage_shared)                                                                  \
-      km_stage_blk<R, F, false><<<G(T_CELL), BLK, lds, s>>>(cs, M(T_CELL), mode, ak, bk, wr,    \
-                                                            epi);                               \
+      km_rk3_blk<R, F, false><<<G(T_CELL), BLK, lds, s>>>(cs, M(T_CELL), rev, keep, 1);         \
     else if (x0->stage_local)                                                                   \
-      km_stage<R, F, true><<<G(T_CELL), BLK, lds, s>>>(cs, M(T_CELL), mode, ak, bk, wr, epi);   \
+      km_rk3<R, F, true><<<G(T_CELL), BLK, lds, s>>>(cs, M(T_CELL), rev, keep, 1);              \
     else                                                                                        \
-      km_stage<R, F, false><<<G(T_CELL), BLK, 0, s>>>(cs, M(T_CELL), mode, ak, bk, wr, epi);    \
+      km_rk3<R, F, false><<<G(T_CELL), BLK, 0, s>>>(cs, M(T_CELL), rev, keep, 1);               \
+    if (b->cnt[T_BF])                                                                           \
+      km_rk3_bcell<R, F><<<G(T_BF), BLK, 0, s>>>(cs, M(T_BF), x0->stage_shared ? 1 : 0, keep, 1); \
   } while (0)
-    switch (x0->p.flux) {
-      case UFX_FLUX_ROE: KMS(1); break;
-      case UFX_FLUX_AUSM: KMS(2); break;
-      case UFX_FLUX_VANLEER: KMS(3); break;
-      default: KMS(4); break;
-    }
-#undef KMS
+  switch (x0->p.flux) {
+    case UFX_FLUX_ROE: KMS(1); break;
+    case UFX_FLUX_AUSM: KMS(2); break;
+    case UFX_FLUX_VANLEER: KMS(3); break;
+    default: KMS(4); break;
   }
+#undef KMS
   km_norm_final<R><<<G(T_CASE), BLK, 0, s>>>(cs, M(T_CASE), k);
   return launch_check();
 }
