@@ -335,7 +335,7 @@ def main_nc(args) -> int:
                          "frac": round(b / (ms_it / 1000.0) / 1e9 / HBM_PEAK_GBS, 4),
                          "launches_per_iteration": round(prof[k][1] / args.steps, 1)}
     dom = max(passes, key=lambda k: passes[k]["ms_per_iteration"])
-    kname = {"lusgs": "k_nc_lusgs_mc" if args.lusgs_order == "multicolour" else "k_nc_lusgs_stream",
+    kname = {"lusgs": "k_nc_lusgs_mc" if args.lusgs_order == "multicolour" else "k_sweep",
              "residual": "k_nc_residual_blk", "gradient": "k_nc_grad_lim",
              "save_old": "k_nc_save_old"}[dom]
     d_ms = passes[dom]["ms_per_iteration"]

@@ -6,6 +6,7 @@
 
 #include "cc_device.h"
 #include "cc_physics.h"
+#include "sweep.h"
 
 namespace ufx {
 
@@ -1664,6 +1665,66 @@ __global__ __launch_bounds__(BLK) void k_lusgs_level(DevT<R> d, Gas<double> g, c
     st4d(d.upper + (size_t)it * 4, o);
   }
 }
+
+// ---- reference-order sweeps in one workgroup (sweep.h)
+constexpr int CC_SW_RING = 1536;  // records in the LDS ring
+
+// lusgs2 and its normal_flux, CCFVM/lusgs.F90:244-310,328-359.  An entry:
+// the outward normal, (face length, 1.5 lambda), the flux of the neighbour's
+// old state (2).
+struct CcSweep {
+  static constexpr int NE = 4;
+  Gas<double> g;
+  const double *cv, *dt, *la;
+  __device__ __forceinline__ double diag(int c) const { return cv[c] / dt[c] + 0.5 * 1.5 * la[c]; }
+  // rho, u, v, p and E + p (the reference forms E as (E / rho) rho)
+  __device__ __forceinline__ void prims(const double* q, double* o) const {
+    double p[5];
+    con2prim(g, q, p);
+    o[0] = p[0];
+    o[1] = p[1];
+    o[2] = p[2];
+    o[3] = p[3];
+    o[4] = q[0] + p[3];
+  }
+  __device__ __forceinline__ void normal(const double* w, double nx, double ny, double* f) const {
+    const double un = w[1] * nx + w[2] * ny;
+    f[0] = w[4] * un;
+    f[1] = w[0] * un;
+    f[2] = f[1] * w[1] + w[3] * nx;
+    f[3] = f[1] * w[2] + w[3] * ny;
+  }
+  __device__ __forceinline__ void entry(const double* q, double l15, double2* en,
+                                        size_t np) const {
+    const double2 n = en[0];
+    double2 dsl = en[np];
+    double w[5], f[4];
+    prims(q, w);
+    normal(w, n.x, n.y, f);
+    dsl.y = l15;
+    en[np] = dsl;
+    en[2 * np] = make_double2(f[0], f[1]);
+    en[3 * np] = make_double2(f[2], f[3]);
+  }
+  __device__ __forceinline__ void term(const double* nb, const double2* e, double* cres) const {
+    const double fo[4] = {e[2].x, e[2].y, e[3].x, e[3].y};
+    double f[4];
+    normal(nb + 4, e[0].x, e[0].y, f);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cres[i] = cres[i] + ((f[i] - fo[i]) * e[1].x - e[1].y * nb[i]);
+  }
+  template <int DIR>
+  __device__ __forceinline__ void update(const double* r, const double* pd, const double* cres,
+                                         double d, double y, double* dq) const {
+    double a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = DIR == 0 ? r[i] - 0.5 * cres[i] : 0.5 * cres[i];
+    sweep_div4(a, d, y, dq);
+    if (DIR == 1)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dq[i] = pd[i] - dq[i];
+  }
+};
 
 // qc = qold + upper, CCFVM/lusgs.F90:314-318.
 template <typename R>

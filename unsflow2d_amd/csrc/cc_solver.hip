@@ -123,6 +123,10 @@ struct ufx_cc {
   // LU-SGS level schedule: cells grouped by level, forward then backward
   int* lv_cells = nullptr;
   std::vector<int> lv_fwd_off, lv_bwd_off;
+  SweepDev sw{};                 // reference-order sweeps in one workgroup (sweep.h)
+  int sw_npass[2] = {0, 0};      // their passes; 0: no plan (the level launches sweep)
+  int sw_nstep[2] = {0, 0};      // and steps
+  int sw_maxe = 0;               // most swept neighbours of a cell
   // multicolour LU-SGS: storage cells by colour, offsets of each colour
   int* mc_cells = nullptr;
   std::vector<int> mc_off;
@@ -576,8 +580,9 @@ int run_stage(ufx_cc* x, DevT<R>& d, int stage, bool norm) {
   return UFX_OK;
 }
 
-// lusgs2, CCFVM/lusgs.F90:207-379: residual, level-scheduled forward and
-// backward sweeps, update.
+// lusgs2, CCFVM/lusgs.F90:207-379: residual, forward and backward sweeps in
+// the reference's order (sweep.h; one launch per level when the context was
+// not made for LU-SGS) or by colour, update.
 template <typename R>
 int run_lusgs(ufx_cc* x, DevT<R>& d) {
   if (int rc = run_residual_full(x, d)) return rc;
@@ -594,6 +599,24 @@ int run_lusgs(ufx_cc* x, DevT<R>& d) {
     LAUNCH(x, UFX_K_OTHER, k_lusgs_final<R>, x->nblk_cell, d);
     return launch_check();
   }
+  if (x->sw_npass[0] > 0) {
+    const CcSweep sc{x->g, d.cv, d.dt, d.la};
+    LAUNCH(x, UFX_K_OTHER, k_sweep_prep<CcSweep>, nblocks(2 * x->noc), sc, x->sw, d.res, d.qold,
+           d.fla, d.err);
+    // (triangles have at most three neighbours to a sweep)
+#define KSW(ME)                                                                                 \
+  do {                                                                                          \
+    LAUNCH(x, UFX_K_OTHER, (k_sweep<CcSweep, ME, false, CC_SW_RING, 0>), 1, sc, x->sw, 0,       \
+           x->sw_npass[0], x->sw_nstep[0], d.qc, d.err);                                        \
+    LAUNCH(x, UFX_K_OTHER, (k_sweep<CcSweep, ME, false, CC_SW_RING, 1>), 1, sc, x->sw,          \
+           x->sw_npass[0], x->sw_npass[1], x->sw_nstep[1], d.qc, d.err);                        \
+  } while (0)
+    if (x->sw_maxe <= 3) KSW(3);
+    else KSW(MAXF);
+#undef KSW
+    return launch_check();
+  }
+  // no plan (a context made for RK3; see create): the levels one by one
   int nlv = (int)x->lv_fwd_off.size() - 1;
   for (int l = 0; l < nlv; ++l) {
     int a = x->lv_fwd_off[l], n = x->lv_fwd_off[l + 1] - a;
@@ -1276,7 +1299,92 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
   int rc = p.precision == UFX_PREC_FP64
                ? build_dev(x, x->d64, m, sl_face, sl_nbr, cnf, lu_face, lu_cnt, sl)
                : build_dev(x, x->d32, m, sl_face, sl_nbr, cnf, lu_face, lu_cnt, sl);
+  if (p.timemode == UFX_TIME_LUSGS && p.lusgs_order == UFX_LUSGS_REFERENCE) {
+    // inside a level the order is free; cells of equal neighbour counts
+    // together let a wave skip the entries that none of its cells has
+    std::vector<int> nlo(noc, 0), nhi(noc, 0);
+    for (int c = 0; c < noc; ++c)
+      for (int j = 0; j < m.c2f_ptr[c + 1] - m.c2f_ptr[c]; ++j) {
+        const int o = nbr_of(c, j);
+        if (o < c) ++nlo[sto[c]];
+        else if (o < noc) ++nhi[sto[c]];
+      }
+    auto sort_levels = [&](const std::vector<int>& off, const std::vector<int>& cnt) {
+      for (size_t l = 0; l + 1 < off.size(); ++l)
+        std::stable_sort(lv_cells.begin() + off[l], lv_cells.begin() + off[l + 1],
+                         [&](int a, int b) { return cnt[a] > cnt[b]; });
+    };
+    sort_levels(x->lv_fwd_off, nlo);
+    sort_levels(x->lv_bwd_off, nhi);
+    const size_t np = 2 * (size_t)noc;
+    std::vector<int> pos(np), out(np), nb;
+    for (size_t s2 = 0; s2 < np; ++s2) pos[(s2 < (size_t)noc ? 0 : noc) + lv_cells[s2]] = (int)s2;
+    std::vector<size_t> eptr(np + 1, 0);
+    std::vector<int2> eo_all;  // (reference face, bit-inverted when the cell is its `out`; neighbour)
+    for (size_t s2 = 0; s2 < np; ++s2) {
+      const int it = lv_cells[s2], c = x->ref_of_sto[it], dir = s2 < (size_t)noc ? 0 : 1;
+      for (int j = 0; j < m.c2f_ptr[c + 1] - m.c2f_ptr[c]; ++j) {
+        const int f = m.c2f[m.c2f_ptr[c] + j], o = nbr_of(c, j);
+        if (dir == 0 ? o < c : (o > c && o < noc)) {
+          eo_all.push_back(make_int2(m.fout[f] == c ? ~f : f, sto[o]));
+          nb.push_back(pos[(size_t)dir * noc + sto[o]]);
+        }
+      }
+      eptr[s2 + 1] = eo_all.size();
+      out[s2] = dir == 0 ? pos[(size_t)noc + it] - noc : it;
+    }
+    const SweepPlan pl = sweep_plan(noc, x->lv_fwd_off, x->lv_bwd_off, eptr, nb, out, CC_SW_RING);
+    for (size_t s2 = 0; s2 < np; ++s2)
+      x->sw_maxe = std::max(x->sw_maxe, (int)(eptr[s2 + 1] - eptr[s2]));
+    const size_t rows = std::max(x->sw_maxe, 3);  // entry rows that the sweeps load
+    const size_t need = np * (rows * (16 * CcSweep::NE + 8) + 16 + 64 + 16) +
+                        (size_t)noc * (32 + 8 * SW_GREC) +
+                        pl.pass.size() * (16 + 4 * SW_WIDTH);
+    size_t mem_free = 0, mem_all = 0;
+    if (hipMemGetInfo(&mem_free, &mem_all) != hipSuccess) {
+      (void)hipGetLastError();
+      mem_free = 0;
+    }
+    // A step takes 0.7 us, a level's launch 7 us: the launches are faster
+    // only where a level is more than ten steps (a level is two or three
+    // steps on a channel of two million triangles).  They also remain where
+    // the plan does not fit the memory or its 32-bit offsets.
+    const size_t steps = (size_t)pl.nstep[0] + pl.nstep[1];
+    const size_t levels = x->lv_fwd_off.size() + x->lv_bwd_off.size() - 2;
+    if (steps <= 10 * levels + 16 && need < mem_free / 2 && np <= ((size_t)1 << 27)) {
+      std::vector<int2> pe(rows * np, make_int2(0, 0));
+      std::vector<double2> ent(rows * CcSweep::NE * np, make_double2(0.0, 0.0));
+      // the face geometry as the face records hold it
+      auto in_r = [&](double v) { return p.precision == UFX_PREC_FP64 ? v : (double)(float)v; };
+      for (size_t s2 = 0; s2 < np; ++s2)
+        for (size_t j = eptr[s2]; j < eptr[s2 + 1]; ++j) {
+          const size_t k = j - eptr[s2];
+          const bool inv = eo_all[j].x < 0;
+          const int f = inv ? ~eo_all[j].x : eo_all[j].x;
+          const double nx = in_r(m.fnx[f]), ny = in_r(m.fny[f]);
+          pe[k * np + s2] = make_int2(x->face_of_ref[f], eo_all[j].y);
+          ent[k * CcSweep::NE * np + s2] = inv ? make_double2(-nx, -ny) : make_double2(nx, ny);
+          ent[(k * CcSweep::NE + 1) * np + s2] = make_double2(in_r(m.farea[f]), 0.0);
+        }
+      SweepDev& w = x->sw;
+      w.np = (int)np;
+      if (!rc) rc = dupload(x, &w.pass, pl.pass);
+      if (!rc) rc = dupload(x, &w.far, pl.far);
+      if (!rc) rc = dupload(x, &w.head, pl.head);
+      if (!rc) rc = dupload(x, &w.pe, pe);
+      if (!rc) rc = dupload(x, &w.ent, ent);
+      if (!rc) rc = dalloc(x, &w.own, 4 * np);
+      if (!rc) rc = dalloc(x, &w.diag, np);
+      if (!rc) rc = dalloc(x, &w.fwd, 4 * (size_t)noc);
+      if (!rc) rc = dalloc(x, &w.rec, (size_t)SW_GREC * (noc + 1));
+      for (int dir = 0; !rc && dir < 2; ++dir) {
+        x->sw_npass[dir] = pl.npass[dir];
+        x->sw_nstep[dir] = pl.nstep[dir];
+      }
+    }
+  }
   if (!rc) rc = dupload(x, &x->lv_cells, lv_cells);
+  x->sw.node = x->lv_cells;
   if (!rc && p.timemode == UFX_TIME_LUSGS && p.lusgs_order == UFX_LUSGS_MULTICOLOUR) {
     // colours of the interior cells (reference numbering) -> storage order;
     // each colour's cells in ascending storage order (compact blocks)

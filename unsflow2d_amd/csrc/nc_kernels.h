@@ -22,6 +22,7 @@
 
 #include "cc_device.h"
 #include "cc_physics.h"
+#include "sweep.h"
 
 namespace ufx {
 
@@ -74,21 +75,6 @@ struct DevNC {
   double* part;  // reduction partials [nblk][4]
   double* scal;  // [0] fres1
   int* err;
-  // level-ordered sweep data (positions: forward levels, then backward)
-  // Streamed sweeps: position s (0 .. 2 nop - 1) is the s-th vertex of the
-  // forward levels then of the backward levels; every array below is
-  // position-major (a wave's lanes read consecutive addresses), with sw_q
-  // entry slots per position for its swept neighbours in edge order.
-  const int* sw_vert;   // [2 nop] vertex of each position
-  const int* sw_cnt;    // [2 nop] swept neighbours of each position
-  const int* sw_nb;     // [sw_q][2 nop] neighbour's position, bit-inverted when the vertex is p2
-  const int2* sw_pe;    // [sw_q][2 nop] (edge, neighbour vertex)
-  const int* sw_d0;     // [2 nop] forward position of the vertex (read by backward positions)
-  double2* sw_ent;      // [sw_q][6][2 nop] (nx,ny) (ds,la_e) F(qold_o) (2) qold_o (2)
-  double2* sw_own;      // [4][2 nop] res (2), qold (2)
-  double* sw_dd;        // [2 nop] diagonal
-  double* sw_dq;        // [2 nop][4] dq of each position
-  int sw_q;             // entry slots per position
   // multicolour sweeps: positions 0 .. nop - 1 are the vertices grouped by
   // colour (ascending vertex number inside a colour); per sweep direction and
   // position, mc_q entry slots (position-major) hold the neighbours of lower
@@ -1134,167 +1120,71 @@ __global__ __launch_bounds__(BLK) void k_nc_lusgs_mc(DevNC d, NCFree g, int s0, 
   st4d(d.mc_dq + (size_t)s * 4, dq);
 }
 
-// ---- level-ordered one-workgroup sweeps
-// A sweep level touches a few hundred vertices scattered over the mesh, and
-// in one workgroup everything it reads enters through one CU, whose address
-// unit handles about one distinct cache line per lane-access of a scattered
-// load.  So the data that does not depend on the sweep is first written in
-// level order by a parallel pass, position-major, and inside the sweep only
-// the swept neighbours' dq (one 32-byte record per position) is gathered;
-// their state is rebuilt as qold_o + dq_o, the same sum that produced it.
-constexpr int SWE = 6;
+// ---- reference-order sweeps in one workgroup (sweep.h)
+// The LDS ring of the last positions' records (with the area of the stored
+// records beside it 147 KB of a CU's 160 KB); 1.4 % to 3 % of the reads of a
+// 180 000-vertex O-grid lie beyond it.
+constexpr int SW_RING = 1536;
+constexpr int SW_ENTRIES = 5;  // 0.1 % of an O-grid's vertices have more swept neighbours
 
-// Per position: the vertex's residual, old state and diagonal; per swept
-// entry: the edge's spectral radius, normalflux of the neighbour's old state
-// (NCFVM/lusgs.f90:62-72) and that old state.  The geometry of the entries
-// (nx, ny, ds) is written once at set-up.
-__global__ __launch_bounds__(BLK) void k_nc_sweep_prep(DevNC d, NCFree g) {
-  const int np = 2 * d.nop;
-  int s = blockIdx.x * BLK + threadIdx.x;
-  if (s >= np) return;
-  const int v = d.sw_vert[s];
-  const double2* r = reinterpret_cast<const double2*>(d.res + (size_t)v * 4);
-  const double2* qo = reinterpret_cast<const double2*>(d.qold + (size_t)v * 4);
-  d.sw_own[s] = r[0];
-  d.sw_own[(size_t)np + s] = r[1];
-  d.sw_own[2 * (size_t)np + s] = qo[0];
-  d.sw_own[3 * (size_t)np + s] = qo[1];
-  d.sw_dd[s] = d.dd[v];
-  const int cnt = d.sw_cnt[s];
-  for (int k = 0; k < cnt; ++k) {
-    const int2 pe = d.sw_pe[(size_t)k * np + s];
-    double2* en = d.sw_ent + (size_t)k * SWE * np + s;
+// NCFVM/lusgs.f90:46-122 and normalflux (:135-155), term for term.  An
+// entry: (nx, ny), (length, 1.5 lambda), normalflux of the neighbour's old
+// state (2); its normal carries the reference's sign (negation commutes with
+// every rounding).
+struct NcSweep {
+  static constexpr int NE = 4;
+  NCFree g;
+  const double* dd;
+  __device__ __forceinline__ double diag(int v) const { return dd[v]; }
+  __device__ __forceinline__ void entry(const double* q, double l15, double2* en,
+                                        size_t np) const {
     const double2 nxy = en[0];
     double2 dsl = en[np];
-    double q[4], f1[4];
-    ld4d(d.qold + (size_t)pe.y * 4, q);
-    nc_normalflux(g, q, nxy.x, nxy.y, dsl.x, f1);
-    dsl.y = d.fla[pe.x];
+    double f[4];
+    nc_normalflux(g, q, nxy.x, nxy.y, dsl.x, f);
+    dsl.y = l15;
     en[np] = dsl;
-    en[2 * (size_t)np] = make_double2(f1[0], f1[1]);
-    en[3 * (size_t)np] = make_double2(f1[2], f1[3]);
-    en[4 * (size_t)np] = make_double2(q[0], q[1]);
-    en[5 * (size_t)np] = make_double2(q[2], q[3]);
+    en[2 * np] = make_double2(f[0], f[1]);
+    en[3 * np] = make_double2(f[2], f[3]);
   }
-}
-
-// One sweep in one workgroup over the level-ordered data.  The loads of the
-// first SWP entry slots of a position are issued together, each under its
-// slot's own k < cnt test.
-constexpr int SWP = 5;
-constexpr int STREAM_THREADS = 512;
-
-struct SwSlot {
-  double2 nxy, dsl, f01, f23, q01, q23;
-  int nb;
-  double dq[4];
+  // rho, u, v, p and E + p of the state q, as normalflux forms them
+  __device__ __forceinline__ void prims(const double* q, double* o) const {
+    double rho = q[1], u = q[2] / q[1], v = q[3] / q[1], et = q[0];
+    double e = et / rho;
+    double qq = u * u + v * v;
+    double p = (g.gamma - 1.0) * (et - 0.5 * rho * qq);
+    double ee = e * rho;
+    o[0] = rho;
+    o[1] = u;
+    o[2] = v;
+    o[3] = p;
+    o[4] = ee + p;
+  }
+  // one swept neighbour (its record nb): normalflux of its new state against
+  // that of its old one (0.5 times a value is exact)
+  __device__ __forceinline__ void term(const double* nb, const double2* e, double* cres) const {
+    const double nx = e[0].x, ny = e[0].y, ds = e[1].x, l15 = e[1].y;
+    const double f1[4] = {e[2].x, e[2].y, e[3].x, e[3].y};
+    const double rho = nb[4], u = nb[5], v = nb[6], p = nb[7];
+    const double un = u * nx + v * ny;
+    const double m = rho * un;
+    const double f2[4] = {nb[8] * un * ds, m * ds, (m * u + p * nx) * ds, (m * v + p * ny) * ds};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      cres[i] = __builtin_fma(0.5, (f2[i] - f1[i]) - l15 * nb[i], cres[i]);
+  }
+  template <int DIR>
+  __device__ __forceinline__ void update(const double* r, const double* pd, const double* cres,
+                                         double d, double y, double* dq) const {
+    double a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = DIR == 0 ? r[i] - cres[i] : cres[i];
+    sweep_div4(a, d, y, dq);
+    if (DIR == 1)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dq[i] = pd[i] - dq[i];
+  }
 };
-
-// The dq of the last SW_RING positions of a sweep is also kept in LDS (a
-// ring indexed by position mod SW_RING, 160 KB, all of a CU's LDS): a
-// neighbour at position o is read from there when o >= lim = level start +
-// level width - SW_RING, which no write of this level or an earlier one has
-// overwritten; the rest (about 3 % on the 2M-vertex O-grid) from HBM.
-constexpr int SW_RING = 5120;
-
-__device__ __forceinline__ void nc_stream_load(const DevNC& d, int np, int s, int k, SwSlot& e,
-                                               const double2* ring, int lim) {
-  e.nb = d.sw_nb[(size_t)k * np + s];
-  const double2* en = d.sw_ent + (size_t)k * SWE * np + s;
-  e.nxy = en[0];
-  e.dsl = en[np];
-  e.f01 = en[2 * (size_t)np];
-  e.f23 = en[3 * (size_t)np];
-  e.q01 = en[4 * (size_t)np];
-  e.q23 = en[5 * (size_t)np];
-  const int o = e.nb >= 0 ? e.nb : ~e.nb;
-  if (o >= lim) {
-    const double2 a = ring[2 * (o % SW_RING)], b = ring[2 * (o % SW_RING) + 1];
-    e.dq[0] = a.x;
-    e.dq[1] = a.y;
-    e.dq[2] = b.x;
-    e.dq[3] = b.y;
-  } else {
-    ld4d(d.sw_dq + (size_t)o * 4, e.dq);
-  }
-}
-
-__device__ __forceinline__ void nc_stream_term(const NCFree& g, const SwSlot& e, double* cres) {
-  const double q[4] = {e.q01.x + e.dq[0], e.q01.y + e.dq[1], e.q23.x + e.dq[2], e.q23.y + e.dq[3]};
-  const double f1[4] = {e.f01.x, e.f01.y, e.f23.x, e.f23.y};
-  double f2[4];
-  nc_normalflux(g, q, e.nxy.x, e.nxy.y, e.dsl.x, f2);
-  double sign = e.nb >= 0 ? 1.0 : -1.0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    cres[i] = cres[i] + 0.5 * (sign * (f2[i] - f1[i]) - 1.5 * e.dsl.y * e.dq[i]);
-}
-
-__device__ __forceinline__ void nc_stream_pos(const DevNC& d, const NCFree& g, int s, int dir,
-                                              double2* ring, int lim) {
-  const int np = 2 * d.nop;
-  const int cnt = d.sw_cnt[s];
-  const double2 r01 = d.sw_own[s], r23 = d.sw_own[(size_t)np + s];
-  const double dd = d.sw_dd[s];
-  double dq0[4];
-  if (dir == 1) ld4d(d.sw_dq + (size_t)d.sw_d0[s] * 4, dq0);
-  SwSlot e[SWP];
-#pragma unroll
-  for (int k = 0; k < SWP; ++k)
-    if (k < cnt) nc_stream_load(d, np, s, k, e[k], ring, lim);
-  double cres[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int k = 0; k < SWP; ++k)
-    if (k < cnt) nc_stream_term(g, e[k], cres);
-  for (int k = SWP; k < cnt; ++k) {
-    SwSlot e2;
-    nc_stream_load(d, np, s, k, e2, ring, lim);
-    nc_stream_term(g, e2, cres);
-  }
-  const double res[4] = {r01.x, r01.y, r23.x, r23.y};
-  double out[4];
-  if (dir == 0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = (-res[i] - cres[i]) / dd;
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = dq0[i] - cres[i] / dd;
-  }
-  st4d(d.sw_dq + (size_t)s * 4, out);
-  ring[2 * (s % SW_RING)] = make_double2(out[0], out[1]);
-  ring[2 * (s % SW_RING) + 1] = make_double2(out[2], out[3]);
-}
-
-// A level's writes go to the slots of positions [b - SW_RING, b + n -
-// SW_RING), below lim, so no read of the level meets them; a level wider
-// than the ring reads only from HBM (lim > b).
-__global__ __launch_bounds__(STREAM_THREADS) void k_nc_lusgs_stream(DevNC d, NCFree g,
-                                                                  const int* off, int nlev,
-                                                                  int dir) {
-  __shared__ double2 ring[2 * SW_RING];
-  for (int l = 0; l < nlev; ++l) {
-    const int b = off[l], n = off[l + 1] - b;
-    const int lim = b + n - SW_RING;
-    for (int t = threadIdx.x; t < n; t += STREAM_THREADS)
-      nc_stream_pos(d, g, b + t, dir, ring, lim);
-    __syncthreads();
-  }
-}
-
-// The sweeps' result: qc = qold + dq of the backward sweep, per backward
-// position (the same sum the sweep used for the neighbours' state).
-__global__ __launch_bounds__(BLK) void k_nc_sweep_final(DevNC d) {
-  const int np = 2 * d.nop;
-  int t = cell_index();
-  if (t >= d.nop) return;
-  const int s = d.nop + t;
-  const int v = d.sw_vert[s];
-  const double2 q01 = d.sw_own[2 * (size_t)np + s], q23 = d.sw_own[3 * (size_t)np + s];
-  double dq[4];
-  ld4d(d.sw_dq + (size_t)s * 4, dq);
-  const double q[4] = {q01.x + dq[0], q01.y + dq[1], q23.x + dq[2], q23.y + dq[3]};
-  st4d(d.qc + (size_t)v * 4, q);
-}
 
 // A whole sweep in one cooperative launch of a few workgroups: the vertices
 // of a level are spread over all of them (so a level's scattered records

@@ -46,6 +46,8 @@ struct ufx_nc {
   std::vector<int> lv_fwd_off, lv_bwd_off;  // offsets into lv_verts
   int *d_fwd_off = nullptr, *d_bwd_off = nullptr;  // the same on the device
   SweepSlot* d_slots = nullptr;             // packed sweep slots, forward then backward
+  SweepDev sw{};                            // one-workgroup sweeps over the level order (sweep.h)
+  int sw_npass[2] = {0, 0}, sw_nstep[2] = {0, 0};  // passes and steps of the forward and the backward sweep
   int nwall = 0;                            // wall edges (bc 1001)
   int* d_wedge = nullptr;                   // their stored edges, in ascending reference order
   std::vector<int> es, es_ref;              // storage slot of each reference edge, and back
@@ -269,20 +271,18 @@ int run_lusgs(ufx_nc* x, double cfl) {
     prof_mark(x, -1);
     return UFX_OK;
   }
-  NLAUNCH(x, NK_LUSGS, k_nc_lusgs_diag, x->nblk, x->d);
   if (x->sweep_mode == 4) {
-    NLAUNCH(x, NK_LUSGS, k_nc_sweep_prep, nblk_of(2 * x->nop), x->d, x->g);
-    for (int dir = 0; dir < 2; ++dir) {
-      const std::vector<int>& off = dir == 0 ? x->lv_fwd_off : x->lv_bwd_off;
-      const int* doff = dir == 0 ? x->d_fwd_off : x->d_bwd_off;
-      prof_mark(x, NK_LUSGS);
-      k_nc_lusgs_stream<<<1, STREAM_THREADS, 0, x->stream>>>(x->d, x->g, doff,
-                                                            (int)off.size() - 1, dir);
-      prof_mark(x, -1);
-    }
-    NLAUNCH(x, NK_LUSGS, k_nc_sweep_final, x->nblk, x->d);
+    // (the residual pass has written the diagonal)
+    const NcSweep sc{x->g, x->d.dd};
+    NLAUNCH(x, NK_LUSGS, k_sweep_prep<NcSweep>, nblk_of(2 * x->nop), sc, x->sw, x->d.res,
+            x->d.qold, x->d.fla, (const int*)nullptr);
+    NLAUNCH(x, NK_LUSGS, (k_sweep<NcSweep, SW_ENTRIES, true, SW_RING, 0>), 1, sc, x->sw, 0,
+            x->sw_npass[0], x->sw_nstep[0], x->d.qc, (const int*)nullptr);
+    NLAUNCH(x, NK_LUSGS, (k_sweep<NcSweep, SW_ENTRIES, true, SW_RING, 1>), 1, sc, x->sw,
+            x->sw_npass[0], x->sw_npass[1], x->sw_nstep[1], x->d.qc, (const int*)nullptr);
     return launch_ok();
   }
+  NLAUNCH(x, NK_LUSGS, k_nc_lusgs_diag, x->nblk, x->d);
   for (int dir = 0; dir < 2; ++dir) {
     const std::vector<int>& off = dir == 0 ? x->lv_fwd_off : x->lv_bwd_off;
     if (x->sweep_mode == 3) {
@@ -744,59 +744,62 @@ int ufx_nc_create(const ufx_mesh* mesh, const ufx_nc_params* prm, ufx_nc** out) 
       sl.cnt = cnt;
     }
     if (!rc && fits) rc = nc_upload(x, &x->d_slots, slots);
-    // position-major data of the streamed one-workgroup sweeps: per
-    // position sw_q slots (the largest swept-neighbour count) holding its
-    // swept neighbours in edge order, with the edge geometry (unused
-    // slots: zeros, never read)
+    // the one-workgroup sweeps over the level order: per position the swept
+    // neighbours in edge order, their passes and LDS slots, and position-major
+    // the edge geometry (unused slots: zeros, never read)
     {
       const size_t np = verts.size();
       std::vector<int> pos(np);  // position of each vertex in each sweep
       for (size_t s = 0; s < np; ++s) pos[(s < (size_t)nop ? 0 : nop) + verts[s]] = (int)s;
-      std::vector<int> sw_cnt(np, 0), sw_d0(np, 0);
+      std::vector<int> nb, out(np);
       std::vector<int2> eo_all;
-      std::vector<size_t> eo_ptr(np + 1, 0);
-      int q = 1;
+      std::vector<size_t> eptr(np + 1, 0);
       for (size_t s = 0; s < np; ++s) {
-        int p = verts[s], dir = s < (size_t)nop ? 0 : 1, cnt = 0;
+        const int p = verts[s], dir = s < (size_t)nop ? 0 : 1;
         for (int j = m.v2f_ptr[p]; j < m.v2f_ptr[p + 1]; ++j) {
-          int e = m.v2f[j];
-          bool first = m.fp1[e] == p;
-          int o = first ? m.fp2[e] : m.fp1[e];
+          const int e = m.v2f[j];
+          const bool first = m.fp1[e] == p;
+          const int o = first ? m.fp2[e] : m.fp1[e];
           if (dir == 0 ? rv[o] < rv[p] : rv[o] > rv[p]) {
+            const int on = pos[(size_t)dir * nop + o];
             eo_all.push_back(make_int2(first ? e : ~e, o));
-            ++cnt;
+            nb.push_back(on);
           }
         }
-        sw_cnt[s] = cnt;
-        sw_d0[s] = pos[p];
-        eo_ptr[s + 1] = eo_all.size();
-        q = std::max(q, cnt);
+        eptr[s + 1] = eo_all.size();
+        out[s] = dir == 0 ? pos[(size_t)nop + p] - nop : p;
       }
-      const size_t nq = (size_t)q;
-      std::vector<int> sw_nb(nq * np, 0);
-      std::vector<int2> sw_pe(nq * np, make_int2(0, 0));
-      std::vector<double2> sw_ent(nq * SWE * np, make_double2(0.0, 0.0));
+      const SweepPlan pl = sweep_plan(nop, cf, cb, eptr, nb, out, SW_RING);
+      const size_t nq = (size_t)pl.q;
+      std::vector<int2> pe(nq * np, make_int2(0, 0));
+      std::vector<double2> ent(nq * 4 * np, make_double2(0.0, 0.0));
       for (size_t s = 0; s < np; ++s)
-        for (size_t j = eo_ptr[s]; j < eo_ptr[s + 1]; ++j) {
-          const size_t k = j - eo_ptr[s];
-          const int2 eo = eo_all[j];
-          const int e = eo.x >= 0 ? eo.x : ~eo.x;
-          const int on = pos[(s < (size_t)nop ? 0 : nop) + eo.y];
-          sw_nb[k * np + s] = eo.x >= 0 ? on : ~on;
-          sw_pe[k * np + s] = make_int2(es[e], eo.y);
-          sw_ent[k * SWE * np + s] = make_double2(m.fnx[e], m.fny[e]);
-          sw_ent[(k * SWE + 1) * np + s] = make_double2(m.farea[e], 0.0);
+        for (size_t j = eptr[s]; j < eptr[s + 1]; ++j) {
+          const size_t k = j - eptr[s];
+          const bool inv = eo_all[j].x < 0;
+          const int e = inv ? ~eo_all[j].x : eo_all[j].x;
+          pe[k * np + s] = make_int2(es[e], eo_all[j].y);
+          ent[k * 4 * np + s] = inv ? make_double2(-m.fnx[e], -m.fny[e])
+                                    : make_double2(m.fnx[e], m.fny[e]);
+          ent[(k * 4 + 1) * np + s] = make_double2(m.farea[e], 0.0);
         }
-      x->d.sw_q = q;
-      x->d.sw_vert = x->lv_verts;
-      if (!rc) rc = nc_upload(x, &x->d.sw_cnt, sw_cnt);
-      if (!rc) rc = nc_upload(x, &x->d.sw_nb, sw_nb);
-      if (!rc) rc = nc_upload(x, &x->d.sw_d0, sw_d0);
-      if (!rc) rc = nc_upload(x, &x->d.sw_pe, sw_pe);
-      if (!rc) rc = nc_upload(x, &x->d.sw_ent, sw_ent);
-      if (!rc) rc = nc_alloc(x, &x->d.sw_own, 4 * np);
-      if (!rc) rc = nc_alloc(x, &x->d.sw_dd, np);
-      if (!rc) rc = nc_alloc(x, &x->d.sw_dq, 4 * np);
+      SweepDev& w = x->sw;
+      w.np = (int)np;
+      w.node = x->lv_verts;
+      for (int dir = 0; dir < 2; ++dir) {
+        x->sw_npass[dir] = pl.npass[dir];
+        x->sw_nstep[dir] = pl.nstep[dir];
+      }
+      if (!rc) rc = nc_upload(x, &w.pass, pl.pass);
+      if (!rc) rc = nc_upload(x, &w.far, pl.far);
+      if (!rc) rc = nc_upload(x, &w.head, pl.head);
+      if (!rc) rc = nc_upload(x, &w.more, pl.slot);
+      if (!rc) rc = nc_upload(x, &w.pe, pe);
+      if (!rc) rc = nc_upload(x, &w.ent, ent);
+      if (!rc) rc = nc_alloc(x, &w.own, 4 * np);
+      if (!rc) rc = nc_alloc(x, &w.diag, np);
+      if (!rc) rc = nc_alloc(x, &w.fwd, 4 * (size_t)nop);
+      if (!rc) rc = nc_alloc(x, &w.rec, (size_t)SW_GREC * (nop + 1));
     }
     if (rc) { ufx_nc_destroy(x); return rc; }
     // sweep form: one workgroup over the level-ordered data (default,
