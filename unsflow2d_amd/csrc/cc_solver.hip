@@ -16,6 +16,7 @@
 
 #include "cc_batch.h"
 #include "cc_kernels.h"
+#include "readback.h"
 #include "ufx_internal.h"
 
 using namespace ufx;
@@ -112,6 +113,8 @@ struct ufx_cc {
   double* cirs_tmp = nullptr;    // [noc][4] the first smoothing sweep's result
   double* bfluxv = nullptr;      // viscous wall force terms [2][nbf]
   std::vector<int> sto_of_ref;   // reference cell -> storage cell (ncell)
+  int* d_sto = nullptr;          // the same on the device
+  Readback rb;
   std::vector<int> ref_of_sto;   // storage cell -> reference cell
   std::vector<int> ref_of_face;  // storage face -> reference face
   std::vector<int> face_of_ref;  // reference face -> storage face
@@ -695,22 +698,12 @@ int get_field(ufx_cc* x, DevT<R>& d, const std::string& n, double* dst) {
   const int noc = x->noc, ncell = x->ncell, nof = x->nof, nop = x->nop;
   const std::vector<int>& sto = x->sto_of_ref;
   if (n == "qc" || n == "qold" || n == "res") {
-    int cnt = n == "qc" ? ncell : noc;
     const double* src = n == "qc" ? d.qc : (n == "qold" ? d.qold : d.res);
-    std::vector<double> t((size_t)cnt * 4);
-    HIPCHK(copy(t.data(), src, t.size() * 8));
-    HIPCHK(hipStreamSynchronize(x->stream));
-    for (int c = 0; c < cnt; ++c)
-      for (int k = 0; k < 4; ++k) dst[(size_t)c * 4 + k] = t[(size_t)sto[c] * 4 + k];
-    return UFX_OK;
+    return read_rows<4>(x->rb, x->device, x->stream, src, x->d_sto, n == "qc" ? ncell : noc, dst);
   }
   if (n == "dt" || n == "la") {
     if (int rc = restore_dtla(x, d)) return rc;
-    std::vector<double> t(noc);
-    HIPCHK(copy(t.data(), n == "dt" ? d.dt : d.la, (size_t)noc * 8));
-    HIPCHK(hipStreamSynchronize(x->stream));
-    for (int c = 0; c < noc; ++c) dst[c] = t[sto[c]];
-    return UFX_OK;
+    return read_rows<1>(x->rb, x->device, x->stream, n == "dt" ? d.dt : d.la, x->d_sto, noc, dst);
   }
   if (n == "qp" || n == "grad" || n == "phi") {
     std::vector<R> rec((size_t)ncell * RW), t((size_t)ncell), gt((size_t)noc * 2);
@@ -1052,6 +1045,7 @@ int ufx_cc_destroy(ufx_cc* x) {
   for (void* p : x->allocs) (void)hipFree(p);
   if (x->d_hist) (void)hipFree(x->d_hist);
   (void)release_chunk(x->chunk);
+  x->rb.release();
   if (x->d_out) (void)hipFree(x->d_out);
   for (hipEvent_t e : x->ev_pool) (void)hipEventDestroy(e);
   if (x->stream) (void)hipStreamDestroy(x->stream);
@@ -1383,6 +1377,8 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
       }
     }
   }
+  if (!rc) rc = dupload(x, &x->d_sto, x->sto_of_ref);
+  (void)x->rb.reserve((size_t)m.ncell() * 32);
   if (!rc) rc = dupload(x, &x->lv_cells, lv_cells);
   x->sw.node = x->lv_cells;
   if (!rc && p.timemode == UFX_TIME_LUSGS && p.lusgs_order == UFX_LUSGS_MULTICOLOUR) {

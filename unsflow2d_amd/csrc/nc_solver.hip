@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "nc_kernels.h"
+#include "readback.h"
 #include "ufx_internal.h"
 
 using namespace ufx;
@@ -38,6 +39,7 @@ struct ufx_nc {
                               // left res and dd by vertex to mc_res, mc_dd
   DevNC d{};
   int nop = 0, nof = 0, nblk = 0;
+  int device = 0;                           // the HIP device the context lives on
   hipStream_t stream = nullptr;
   std::vector<void*> allocs;
   double* d_hist = nullptr;
@@ -52,6 +54,8 @@ struct ufx_nc {
   int* d_wedge = nullptr;                   // their stored edges, in ascending reference order
   std::vector<int> es, es_ref;              // storage slot of each reference edge, and back
   std::vector<int> rv, sv;                  // reference vertex of each storage slot, and back
+  int* d_sto = nullptr;                     // sv on the device
+  Readback rb;
   double *d_fe = nullptr, *d_cp = nullptr;  // [nwall][2] force terms, [nwall] -Cp
   int sweep_mode = 4;                       // 0 graph of level launches, 1 level launches, 2 one workgroup, 3 cooperative grid, 4 level-ordered one workgroup
   int grid_wgs = 8;                         // workgroups of the cooperative sweep
@@ -471,6 +475,7 @@ int ufx_nc_destroy(ufx_nc* x) {
   if (x->stream) (void)hipStreamSynchronize(x->stream);
   for (void* p : x->allocs) (void)hipFree(p);
   if (x->d_hist) (void)hipFree(x->d_hist);
+  x->rb.release();
   for (hipEvent_t e : x->ev) (void)hipEventDestroy(e);
   if (x->sweep_exec) (void)hipGraphExecDestroy(x->sweep_exec);
   if (x->sweep_graph) (void)hipGraphDestroy(x->sweep_graph);
@@ -523,7 +528,8 @@ int ufx_nc_create(const ufx_mesh* mesh, const ufx_nc_params* prm, ufx_nc** out) 
   x->nop = nop;
   x->nof = nof;
   x->nblk = nblk_of(nop);
-  if (hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking) != hipSuccess) {
+  if (hipGetDevice(&x->device) != hipSuccess ||
+      hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking) != hipSuccess) {
     set_error("hipStreamCreate failed");
     delete x;
     return UFX_ERR_HIP;
@@ -943,6 +949,8 @@ int ufx_nc_create(const ufx_mesh* mesh, const ufx_nc_params* prm, ufx_nc** out) 
     }
     NUP(vqp, q64); NUP(vphc, p64); NUP(vxy, x64);
   }
+  if (!rc) rc = nc_upload(x, &x->d_sto, sv);
+  (void)x->rb.reserve((size_t)nop * 32);
   NUP(qc, qc); NUP(cv, m.pcv); NUP(ebc, ebc); NUP(vref, rv);
   NUP(bedge, bedge); NUP(bkind, bkind); NAL(bclos, 10 * bedge.size());
   NUP(be_ptr, be_ptr); NUP(be_edge, be_edge); NUP(sl_loc, sl_loc);
@@ -1132,12 +1140,8 @@ int ufx_nc_get(ufx_nc* x, const char* name, double* dst) {
   // per-vertex arrays (w values each) from storage slots to the reference's
   // vertex numbering
   auto vertex_array = [&](const double* src, int w) -> int {
-    std::vector<double> t((size_t)w * nop);
-    NCCHK(hipMemcpyAsync(t.data(), src, t.size() * 8, hipMemcpyDeviceToHost, x->stream));
-    NCCHK(hipStreamSynchronize(x->stream));
-    for (int p = 0; p < nop; ++p)
-      for (int k = 0; k < w; ++k) dst[(size_t)x->rv[p] * w + k] = t[(size_t)p * w + k];
-    return UFX_OK;
+    return w == 4 ? read_rows<4>(x->rb, x->device, x->stream, src, x->d_sto, nop, dst)
+                  : read_rows<1>(x->rb, x->device, x->stream, src, x->d_sto, nop, dst);
   };
   if (n == "qc") return vertex_array(x->d.qc, 4);
   if (n == "qold") {

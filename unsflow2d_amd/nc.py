@@ -167,7 +167,7 @@ class NCSolver:
     def get(self, name):
         n = self.counts["nof"] if name == "fc_la" else self.counts["nop"]
         w = self.SHAPES.get(name, 1)
-        out = np.zeros((n, w) if w > 1 else n)
+        out = np.empty((n, w) if w > 1 else n)
         _check(lib.ufx_nc_get(self._h, name.encode(), _d(out)))
         return out
 
