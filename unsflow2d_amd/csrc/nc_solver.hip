@@ -161,7 +161,8 @@ int run_grad_lim_r(ufx_nc* x) {
 }
 
 // fvresidual (gradient, limiter, edge fluxes, time step); mode 1 fuses the
-// RK stage update with coefficients (ak, bk)
+// RK stage update with coefficients (ak, bk), mode 3 the three updates of a
+// whole RK3 iteration
 template <typename R>
 int run_fvresidual_r(ufx_nc* x, double cfl, int mode, double ak, double bk) {
   if (int rc = run_grad_lim_r<R>(x)) return rc;
@@ -1074,8 +1075,7 @@ int ufx_nc_iterate(ufx_nc* x, int iter0, int niter, double* hist) {
     x->cfl = cfl;
     if (int rc = run_save_old(x, true)) return rc;
     if (x->prm.timemode == UFX_TIME_RK3) {
-      for (int s = 1; s <= 3; ++s)
-        if (int rc = ufx_nc_rk_stage(x, s, cfl)) return rc;
+      if (int rc = run_fvresidual(x, cfl, 3, 0.0, 0.0)) return rc;
     } else {
       if (int rc = run_lusgs(x, cfl)) return rc;
     }
