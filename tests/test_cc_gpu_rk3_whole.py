@@ -73,3 +73,25 @@ def test_whole_iterations_equal_the_routines(mesh, form, precision, tol):
         for a, b in zip(*out):
             assert np.all(np.isfinite(b))
             assert relerr(a, b) <= tol
+
+
+# A launch of both kinds of cells takes up to 512 blocks of 256 (FP64 gather
+# form: those of the boundary cells, 64 to a block, counted in): 485, 527 and
+# 514 blocks of cells and boundary cells, so that each form is on either side.
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("mixed", 1e-6)])
+@pytest.mark.parametrize("nx,ny", [(240, 250), (256, 255), (257, 256)])
+def test_one_and_two_launches(nx, ny, precision, tol):
+    from unsflow2d_amd import cc, meshgen
+    m = cc.Mesh.from_raw(meshgen.bump_channel(nx, ny, 7, h=0.05))
+    for form in ("gather_lds", "shared", "gather", "shared_lds"):
+        print(f"case: whole rk3 vs routines, {nx}x{ny} {form} {precision}", flush=True)
+        out = []
+        for whole in (True, False):
+            s = cc.Solver(m, cc.Config(mach=0.55, aoa_deg=1.0, precision=precision))
+            s.set_stage_form(form)
+            s.keep_residual(True)
+            h = s.iterate(3) if whole else routines(s, 3)
+            out.append([h, s.get("qc"), s.get("res"), s.get("phi")])
+        for a, b in zip(*out):
+            assert np.all(np.isfinite(b))
+            assert relerr(a, b) <= tol

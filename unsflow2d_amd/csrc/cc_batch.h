@@ -105,7 +105,9 @@ __global__ __launch_bounds__(BLK) void km_rk3(const CaseDesc<R>* cs, const int4*
   int c;
   const VBlock vb = case_block_dir(map, c, rev != 0);
   const CaseDesc<R> e = cs[c];
-  rk3_body<R, FLUX, SL>(e.d, vb, e.gr, e.g, rev, write_res, epi);
+  Rk3Acc acc;
+  rk3_body<R, FLUX, SL>(e.d, vb, e.gr, e.g, rev, write_res, epi, acc);
+  rk3_reduce<R>(e.d, vb.b, epi, acc);
 }
 
 template <typename R, int FLUX, bool SL>
@@ -114,7 +116,9 @@ __global__ __launch_bounds__(BLK) void km_rk3_blk(const CaseDesc<R>* cs, const i
   int c;
   const VBlock vb = case_block_dir(map, c, rev != 0);
   const CaseDesc<R> e = cs[c];
-  rk3_blk_body<R, FLUX, SL>(e.d, vb, e.gr, e.g, rev, write_res, epi);
+  Rk3Acc acc;
+  rk3_blk_body<R, FLUX, SL>(e.d, vb, e.gr, e.g, rev, write_res, epi, acc);
+  rk3_reduce<R>(e.d, vb.b, epi, acc);
 }
 
 // one block per case; history slot k of every case

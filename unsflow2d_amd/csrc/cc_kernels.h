@@ -651,10 +651,12 @@ struct BndOpts {
 // (record `own`), farfield state or wall ghost (built from the inner cell's
 // current conserved state, state(i)), flux F, ghost update and, for walls,
 // the momentum flux of the force sums.  F = 0 for other boundary kinds.
-// Returns false when the Roe average fails.
+// Returns false when the Roe average fails; gp4: the ghost's primitives as
+// stored (untouched for other kinds).
 template <typename R, int FLUX, typename State>
 __device__ __forceinline__ bool bface_one(const DevT<R>& d, const BndOpts& bo, int bc, int k,
-                                          int f, const R* own, State&& state, double* F) {
+                                          int f, const R* own, State&& state, double* F,
+                                          R* gp4) {
   constexpr int RW = Layout<R>::RW, FW = Layout<R>::FW;
   const Gas<double>& g = bo.g;
 #pragma unroll
@@ -717,7 +719,8 @@ __device__ __forceinline__ bool bface_one(const DevT<R>& d, const BndOpts& bo, i
     d.bflux[d.nbf + k] = F[3];
   }
   st4d(d.qc + (size_t)gh * 4, gq);
-  R gp4[4] = {(R)gp[0], (R)gp[1], (R)gp[2], (R)gp[3]};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) gp4[i] = (R)gp[i];
   stv<R, 4>(d.rec + (size_t)gh * RW + R_QP, gp4);
   d.qT[gh] = (R)gp[4];
   return ok;
@@ -736,8 +739,9 @@ __device__ __forceinline__ void bface_body(const DevT<R>& d, VBlock vb, Gas<doub
   R own[RW];
   ldv<R, RW>(d.rec + (size_t)c * RW, own);
   double F[4];
+  R gp4[4];
   if (!bface_one<R, FLUX>(d, bo, d.fbc[k], k, d.bface[k], own,
-                          [&](int i) { return d.qc[(size_t)c * 4 + i]; }, F))
+                          [&](int i) { return d.qc[(size_t)c * 4 + i]; }, F, gp4))
     set_err(d, DERR_ROE, k);
   st4d(d.bres + (size_t)k * 4, F);
 }
@@ -893,44 +897,45 @@ __device__ __forceinline__ void stage_end(const DevT<R>& d, int c, int op, doubl
 // into the records and qT, which other cells are still gathering, and which
 // stay the reference's qp until then), the positivity note for the next
 // iteration (err[1], moved up by the norm) and the block's partial of the
-// limiter's global range over its cells and, with GHOSTS, the ghosts of
-// their boundary faces (which the same thread has written).  Called by every
-// thread of the block; `have`: the thread's cell c is interior, its new state
-// is q and its squared residual sq.
-template <typename R, bool GHOSTS>
-__device__ __forceinline__ void rk3_finish(const DevT<R>& d, int slot, const Gas<double>& g, int c,
-                                           bool have, const double* q, double sq, int epi) {
-  constexpr int RW = Layout<R>::RW;
-  __shared__ double shr[9][BLK / 64];
-  double mx[4], mn[4];
+// limiter's global range over its cells and the ghosts of their boundary
+// faces.
+struct Rk3Acc {  // a thread's part
+  double mx[4], mn[4], sq = 0.0;
+  __device__ __forceinline__ Rk3Acc() {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) { mx[k] = -INFINITY; mn[k] = INFINITY; }
-  if (have && epi) {
-    double p[5];
-    con2prim(g, q, p);
-    R q4[4];
+    for (int k = 0; k < 4; ++k) { mx[k] = -INFINITY; mn[k] = INFINITY; }
+  }
+  template <typename R>
+  __device__ __forceinline__ void range(const R* q4) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) q4[k] = (R)p[k];
-    stv<R, 4>(d.qpc + (size_t)c * 4, q4);
-    d.qTc[c] = (R)p[4];
-    if (p[0] <= 0.0 || p[3] <= 0.0) atomicMin(&d.err[1], d.cref[c] + 1);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) mx[k] = mn[k] = (double)q4[k];
-    if (GHOSTS) {
-      const int info = ld_nt(d.cnf + c), nf = info & 0xff, nb = info >> 8;
-      for (int s = nf - nb; s < nf; ++s) {
-        const int gh = ld_nt(d.sl_nbr + s * d.noc + c);
-        R gq[4];
-        ldv<R, 4>(d.rec + (size_t)gh * RW + R_QP, gq);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const double v = (double)gq[k];
-          mx[k] = v > mx[k] ? v : mx[k];
-          mn[k] = v < mn[k] ? v : mn[k];
-        }
-      }
+    for (int k = 0; k < 4; ++k) {
+      const double v = (double)q4[k];
+      mx[k] = v > mx[k] ? v : mx[k];
+      mn[k] = v < mn[k] ? v : mn[k];
     }
   }
+};
+// Interior cell c, its new state q.
+template <typename R>
+__device__ __forceinline__ void rk3_note(const DevT<R>& d, const Gas<double>& g, int c,
+                                         const double* q, Rk3Acc& acc) {
+  double p[5];
+  con2prim(g, q, p);
+  R q4[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) q4[k] = (R)p[k];
+  stv<R, 4>(d.qpc + (size_t)c * 4, q4);
+  d.qTc[c] = (R)p[4];
+  if (p[0] <= 0.0 || p[3] <= 0.0) atomicMin(&d.err[1], d.cref[c] + 1);
+  acc.range(q4);
+}
+// Called by every thread of the block.
+template <typename R>
+__device__ __forceinline__ void rk3_reduce(const DevT<R>& d, int slot, int epi, Rk3Acc& acc) {
+  __shared__ double shr[9][BLK / 64];
+  double* mx = acc.mx;
+  double* mn = acc.mn;
+  double sq = acc.sq;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     sq = sq + __shfl_xor(sq, off);
@@ -1040,7 +1045,8 @@ __device__ __forceinline__ int bc_index(const DevT<R>& d, int b, int c) {
 
 template <typename R, int FLUX, bool SL>
 __device__ __forceinline__ void rk3_body(const DevT<R>& d, VBlock vb, const Gas<R>& gr,
-                                         const Gas<double>& g, int rev, int write_res, int epi) {
+                                         const Gas<double>& g, int rev, int write_res, int epi,
+                                         Rk3Acc& acc) {
   extern __shared__ double lds_raw[];
   R* srec = reinterpret_cast<R*>(lds_raw);  // [BLK][RW] when SL
   const int base = xcd_block_dir(vb.b, vb.n, rev != 0) * BLK;
@@ -1049,7 +1055,6 @@ __device__ __forceinline__ void rk3_body(const DevT<R>& d, VBlock vb, const Gas<
     stage_block_recs(d, srec, base, min(BLK, d.noc - base));
     __syncthreads();
   }
-  double sq = 0.0, q[4] = {0.0, 0.0, 0.0, 0.0};
   const int info = c < d.noc && !d.err[0] ? d.cnf[c] : -1;
   const bool have = info >= 0 && (info >> 8) == 0;
   // the cells with boundary faces: their interior fluxes for k_rk3_bcell in
@@ -1060,46 +1065,54 @@ __device__ __forceinline__ void rk3_body(const DevT<R>& d, VBlock vb, const Gas<
     const int ekey =
         gather_residual<R, FLUX, SL, false>(d, srec, base, c, gr, r, keep, 4 * (size_t)d.nbc);
     if (ekey != INT_MAX) set_err(d, DERR_ROE, ekey);
-    if (have) sq = rk3_cell<R>(d, c, r, write_res, q);
+    if (have) {
+      double q[4];
+      acc.sq = rk3_cell<R>(d, c, r, write_res, q);
+      if (epi) rk3_note<R>(d, g, c, q, acc);
+    }
   }
-  rk3_finish<R, false>(d, vb.b, g, c, have, q, sq, epi);
 }
 template <typename R, int FLUX, bool SL>
 __global__ __launch_bounds__(BLK) void k_rk3(DevT<R> d, Gas<R> gr, Gas<double> g, int rev,
                                              int write_res, int epi) {
-  rk3_body<R, FLUX, SL>(d, hw_block(), gr, g, rev, write_res, epi);
+  Rk3Acc acc;
+  const VBlock vb = hw_block();
+  rk3_body<R, FLUX, SL>(d, vb, gr, g, rev, write_res, epi, acc);
+  rk3_reduce<R>(d, vb.b, epi, acc);
 }
 
-// The cells with boundary faces, BC_CELLS to a block, after the block's other
-// cells.  stored: their interior fluxes were left in bcF by the pass over the
-// other cells (the block-shared form, and the mixed form: an FP32 flux
+// The cells t0 .. t1 - 1 of the list of cells with boundary faces, BC_CELLS at
+// a time.  stored: their interior fluxes were left in bcF by the pass over
+// the other cells (the block-shared form, and the mixed form: an FP32 flux
 // evaluated here could round differently than in a routine's residual), else
-// they are evaluated here.  The kernel is a chain of latencies (a few dozen blocks), so
-// its work is spread over the lanes, its lists are packed (bc_tab: one load
+// they are evaluated here.  This is a chain of latencies, so its work is
+// spread over the lanes, its lists are packed (bc_tab: one load
 // where cnf, sl_nbr, sl_face and fbc would be a chain of three) and its code
 // kept short: one wave per face slot
 // evaluates that slot's fluxes, the first wave sums them and applies the
 // stage updates, one lane per cell.  Interior and farfield fluxes do not
-// change over the stages; a wall's is evaluated in each.  slot0: the blocks'
-// first slot among the partials.  A wall face failing in a later stage counts
-// after every failure of the earlier ones (the key gets the stage in front,
-// see set_err).
+// change over the stages; a wall's is evaluated in each.  A wall face failing
+// in a later stage counts after every failure of the earlier ones (the key
+// gets the stage in front, see set_err).
 constexpr int BC_CELLS = BLK / MAXF;
 template <typename R, int FLUX>
-__device__ __forceinline__ void rk3_bcell_body(const DevT<R>& d, VBlock vb, int slot0,
-                                               const Gas<R>& gr, const BndOpts& bo, int stored,
-                                               int write_res, int epi) {
+__device__ __forceinline__ void rk3_bcells(const DevT<R>& d, int t0, int t1, const Gas<R>& gr,
+                                           const BndOpts& bo, int stored, int write_res, int epi,
+                                           Rk3Acc& acc) {
   static_assert(BC_CELLS == 64, "one wave per face slot");
   constexpr int RW = Layout<R>::RW, FW = Layout<R>::FW;
   __shared__ double s_F[MAXF][4][BC_CELLS];
   __shared__ double s_q[4][BC_CELLS];
   __shared__ int s_in[MAXF][BC_CELLS];  // the cell is the slot's face's `in`
   const int l = threadIdx.x % BC_CELLS, s = threadIdx.x / BC_CELLS;
-  const int t = vb.b * BC_CELLS + l;
-  const bool run = t < d.nbc && !d.err[0];
-  const int tc = min(t, d.nbc - 1), c = d.bc_cell[tc];
+#pragma unroll 1
+  for (; t0 < t1; t0 += BC_CELLS) {
+  const int t = t0 + l;
+  const bool run = t < t1 && !d.err[0];
+  const int tc = min(t, t1 - 1), c = d.bc_cell[tc];
   const int4 tab = d.bc_tab[(size_t)s * d.nbc + tc];
   const int nf = tab.w & 0xff, ni = nf - (tab.w >> 8), f = tab.y;
+  R gp4[4];    // and its ghost's primitives
   R own[RW];
   int k = -1;  // this slot's boundary face
   if (run && s < ni) {
@@ -1120,10 +1133,11 @@ __device__ __forceinline__ void rk3_bcell_body(const DevT<R>& d, VBlock vb, int 
     s_in[s][l] = in_side;
   } else if (run && s < nf) {
     ldv<R, RW>(d.rec + (size_t)c * RW, own);
+    ldv<R, 4>(d.rec + (size_t)tab.x * RW + R_QP, gp4);
     k = tab.x - d.noc;
   }
   const bool have = run && s == 0;
-  double sq = 0.0, q[4] = {0.0, 0.0, 0.0, 0.0}, q0[4] = {0.0, 0.0, 0.0, 0.0}, r[4], dta = 0.0;
+  double q[4] = {0.0, 0.0, 0.0, 0.0}, q0[4] = {0.0, 0.0, 0.0, 0.0}, r[4], dta = 0.0;
   if (have) {
     dta = d.dta[c];
     ld4d(d.qc + (size_t)c * 4, q0);
@@ -1135,7 +1149,8 @@ __device__ __forceinline__ void rk3_bcell_body(const DevT<R>& d, VBlock vb, int 
   for (int st = 0; st < 3; ++st) {
     if (k >= 0 && (st == 0 || tab.z == WALL)) {
       double F[4];
-      if (!bface_one<R, FLUX>(d, bo, tab.z, k, f, own, [&](int i) { return s_q[i][l]; }, F))
+      if (!bface_one<R, FLUX>(d, bo, tab.z, k, f, own, [&](int i) { return s_q[i][l]; }, F,
+                             gp4))
         set_err(d, DERR_ROE, st * (d.nbf + d.nof) + k);
 #pragma unroll
       for (int i = 0; i < 4; ++i) s_F[s][i][l] = F[i];
@@ -1165,10 +1180,25 @@ __device__ __forceinline__ void rk3_bcell_body(const DevT<R>& d, VBlock vb, int 
   if (have) {
     st4d(d.qc + (size_t)c * 4, q);
     if (write_res) st4d(d.res + (size_t)c * 4, r);
+    double sq = 0.0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) sq = sq + r[i] * r[i];
+    acc.sq = acc.sq + sq;
+    if (epi) rk3_note<R>(d, bo.g, c, q, acc);
   }
-  rk3_finish<R, true>(d, slot0 + vb.b, bo.g, c, have, q, sq, epi);
+  if (k >= 0) acc.range(gp4);
+  }
+}
+// BC_CELLS to a block, after k_rk3 or k_rk3_blk.  slot0: the blocks' first
+// slot among the partials.
+template <typename R, int FLUX>
+__device__ __forceinline__ void rk3_bcell_body(const DevT<R>& d, VBlock vb, int slot0,
+                                               const Gas<R>& gr, const BndOpts& bo, int stored,
+                                               int write_res, int epi) {
+  const int t0 = vb.b * BC_CELLS;
+  Rk3Acc acc;
+  rk3_bcells<R, FLUX>(d, t0, min(t0 + BC_CELLS, d.nbc), gr, bo, stored, write_res, epi, acc);
+  rk3_reduce<R>(d, slot0 + vb.b, epi, acc);
 }
 template <typename R, int FLUX>
 __global__ __launch_bounds__(BLK) void k_rk3_bcell(DevT<R> d, int slot0, Gas<R> gr, BndOpts bo,
@@ -1292,12 +1322,11 @@ __global__ __launch_bounds__(BLK) void k_stage_blk(DevT<R> d, Gas<R> gr, int op,
 template <typename R, int FLUX, bool SL>
 __device__ __forceinline__ void rk3_blk_body(const DevT<R>& d, VBlock vb, const Gas<R>& gr,
                                              const Gas<double>& g, int rev, int write_res,
-                                             int epi) {
+                                             int epi, Rk3Acc& acc) {
   const int b = xcd_block_dir(vb.b, vb.n, rev != 0);
   bool run;
   const R* fl = blk_fluxes<R, FLUX, SL>(d, b, gr, &run);
   const int c = b * BLK + threadIdx.x;
-  double sq = 0.0, q[4] = {0.0, 0.0, 0.0, 0.0};
   const int info = run && c < d.noc ? ld_nt(d.cnf + c) : -1;
   const bool have = info >= 0 && (info >> 8) == 0;
   if (info >= 0 && !have) {
@@ -1312,14 +1341,60 @@ __device__ __forceinline__ void rk3_blk_body(const DevT<R>& d, VBlock vb, const 
   if (have) {
     double r[4];
     blk_residual<R, false>(d, c, info, fl, r);
-    sq = rk3_cell<R>(d, c, r, write_res, q);
+    double q[4];
+    acc.sq = rk3_cell<R>(d, c, r, write_res, q);
+    if (epi) rk3_note<R>(d, g, c, q, acc);
   }
-  rk3_finish<R, false>(d, vb.b, g, c, have, q, sq, epi);
 }
 template <typename R, int FLUX, bool SL>
 __global__ __launch_bounds__(BLK) void k_rk3_blk(DevT<R> d, Gas<R> gr, Gas<double> g, int rev,
                                                  int write_res, int epi) {
-  rk3_blk_body<R, FLUX, SL>(d, hw_block(), gr, g, rev, write_res, epi);
+  Rk3Acc acc;
+  const VBlock vb = hw_block();
+  rk3_blk_body<R, FLUX, SL>(d, vb, gr, g, rev, write_res, epi, acc);
+  rk3_reduce<R>(d, vb.b, epi, acc);
+}
+
+// Both kinds of cells in one launch.  FP64 gather form (nothing of one kind
+// waits for the other): the blocks of the cells with boundary faces come
+// first, being the longer chain.  The other forms: each block goes on with
+// the boundary cells among its own once their interior fluxes are in bcF.
+// Both chains are latencies on meshes this kernel takes: 20 000 cells in FP64
+// take 15 us where the two launches took 11 and 15, 100 000 in the mixed form
+// 23 us where they took 13 and 14.
+template <typename R, int FLUX, bool SL, bool SHARED>
+__global__ __launch_bounds__(BLK, 2) void k_rk3_all(DevT<R> d, Gas<R> gr, Gas<double> g,
+                                                    BndOpts bo, int nblk_cell, int rev,
+                                                    int write_res, int epi) {
+  Rk3Acc acc;
+  const int nbb = (d.nbc + BC_CELLS - 1) / BC_CELLS;
+  if constexpr (sizeof(R) == 8 && !SHARED) {
+    int b = (int)blockIdx.x;
+    if (b < nbb) {
+      rk3_bcells<R, FLUX>(d, b * BC_CELLS, min((b + 1) * BC_CELLS, d.nbc), gr, bo, 0, write_res,
+                          epi, acc);
+      b += nblk_cell;
+    } else {
+      b -= nbb;
+      rk3_body<R, FLUX, SL>(d, VBlock{b, nblk_cell}, gr, g, rev, write_res, epi, acc);
+    }
+    rk3_reduce<R>(d, b, epi, acc);
+  } else {
+    const VBlock vb = hw_block();
+    if constexpr (SHARED) rk3_blk_body<R, FLUX, SL>(d, vb, gr, g, rev, write_res, epi, acc);
+    else rk3_body<R, FLUX, SL>(d, vb, gr, g, rev, write_res, epi, acc);
+    __syncthreads();
+    const int b = xcd_block_dir(vb.b, vb.n, rev != 0);
+    rk3_bcells<R, FLUX>(d, d.bc_ptr[b], b + 1 < vb.n ? d.bc_ptr[b + 1] : d.nbc, gr, bo, 1,
+                        write_res, epi, acc);
+    rk3_reduce<R>(d, vb.b, epi, acc);
+    // the slots that the boundary cells have in two launches: nothing
+    for (int i = vb.b; i < nbb; i += vb.n) {
+      if (threadIdx.x == 0) d.part[nblk_cell + i] = 0.0;
+      if (threadIdx.x < 8)
+        d.rpart[(size_t)(nblk_cell + i) * 8 + threadIdx.x] = threadIdx.x < 4 ? -INFINITY : INFINITY;
+    }
+  }
 }
 
 // Sutherland viscosity of the interior cells from the current state,

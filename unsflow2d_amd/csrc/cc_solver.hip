@@ -204,6 +204,9 @@ int nblocks(int n) { return std::max(1, (n + BLK - 1) / BLK); }
 // LDS a residual-stage block may take (the kernels are launched with it as
 // dynamic shared memory)
 constexpr size_t STAGE_LDS_MAX = 64 * 1024;
+// k_rk3_all: blocks of one launch at most, and its LDS beside the stage's
+constexpr int RK3_ALL_BLOCKS = 512;
+constexpr size_t RK3_ALL_LDS = 12 * 1024;
 
 int launch_check() {
   hipError_t e = hipGetLastError();
@@ -473,16 +476,35 @@ int run_stage_kernel(ufx_cc* x, DevT<R>& d, int op, int rev, double ak, double b
   return launch_check();
 }
 
-// The three stages of a whole inviscid RK3 iteration (k_rk3 and
-// k_rk3_bcell): the cells without boundary faces, then those with.  epi: also
-// the next iteration's primitives.
+// The three stages of a whole inviscid RK3 iteration: the cells without
+// boundary faces and those with, in one launch (k_rk3_all) or in two (k_rk3
+// or k_rk3_blk, then k_rk3_bcell).  epi: also the next iteration's primitives.
 template <typename R>
 int run_rk3(ufx_cc* x, DevT<R>& d, int write_res, int epi) {
   const Gas<R>& gr = gas_of<R>(x);
   const int rev = (x->stage_rev >> 1) & 1;
   const BndOpts bo{x->g, 0, x->p.iwall, x->p.t_wall};
+  // One launch for both kinds of cells while every block of it is resident at
+  // once: two to a CU, with the boundary cells' registers (200 and more; the
+  // other cells alone need 60 to 130 and fill a large mesh's CUs with four to
+  // eight blocks, whose pass takes 120 to 190 us on two million cells, beside
+  // which the boundary cells' 15 us matter little).
+  const bool split64 = sizeof(R) == 8 && !x->stage_shared;
+  const int all = x->nblk_cell + (split64 ? x->nblk_bc : 0);
+  const bool one = x->nblk_bc > 0 && all <= RK3_ALL_BLOCKS &&
+                   x->stage_lds + RK3_ALL_LDS <= STAGE_LDS_MAX;
+#define KA(F, SL, SH)                                                                           \
+  LAUNCH_LDS(x, UFX_K_STAGE, (k_rk3_all<R, F, SL, SH>), all, x->stage_lds, d, gr, x->g, bo,     \
+             x->nblk_cell, rev, write_res, epi)
 #define KR(F)                                                                                   \
   do {                                                                                          \
+    if (one) {                                                                                  \
+      if (x->stage_shared && x->stage_local) KA(F, true, true);                                 \
+      else if (x->stage_shared) KA(F, false, true);                                             \
+      else if (x->stage_local) KA(F, true, false);                                              \
+      else KA(F, false, false);                                                                 \
+      break;                                                                                    \
+    }                                                                                           \
     if (x->stage_shared && x->stage_local)                                                      \
       LAUNCH_LDS(x, UFX_K_STAGE, (k_rk3_blk<R, F, true>), x->nblk_cell, x->stage_lds, d, gr,    \
                  x->g, rev, write_res, epi);                                                    \
@@ -506,6 +528,7 @@ int run_rk3(ufx_cc* x, DevT<R>& d, int write_res, int epi) {
     default: KR(4); break;
   }
 #undef KR
+#undef KA
   return launch_check();
 }
 
