@@ -181,6 +181,35 @@ __device__ __forceinline__ void stv(R* __restrict__ p, const R* v) {
   }
 }
 
+// A wave's records of W values, one per lane (`own`), to rows row0 .. row0 +
+// nrows - 1 of rec, as whole lines.  Stored by the lanes themselves, each
+// instruction writes 16 bytes to each of 64 rows: many times the requests,
+// and lines that L2 gets in pieces.  So the rows pass through the wave's part
+// of LDS and leave it in memory order, N rows at a time (fewer take less LDS,
+// more a shorter chain).  On two million nodes: the cell-centred gradient pass
+// 217 -> 172 us in FP64 and 122 -> 100 us in the mixed form, the
+// vertex-centred one 274 -> 235 us in FP64.
+template <typename R, int W, int N>
+__device__ __forceinline__ void store_records(R* rec, int row0, int nrows, const R* own, R* lds) {
+  constexpr int P = W * (int)sizeof(R) / 16;  // 16-byte pieces of a record
+  static_assert(P * 16 == W * (int)sizeof(R), "records are 16-byte multiples");
+  const int lane = (int)threadIdx.x % 64;
+#pragma unroll
+  for (int r0 = 0; r0 < 64; r0 += N) {
+    if (lane / N == r0 / N) stv<R, W>(lds + (lane % N) * W, own);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int n = min(max(nrows - r0, 0), N) * P;
+    const int4* src = reinterpret_cast<const int4*>(lds);
+    int4* dst = reinterpret_cast<int4*>(rec + (size_t)(row0 + r0) * W);
+#pragma unroll
+    for (int i = 0; i < (N * P + 63) / 64; ++i)
+      if (lane + 64 * i < n) dst[lane + 64 * i] = src[lane + 64 * i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 __device__ __forceinline__ void ld4d(const double* p, double* o) {
   const double2* q = reinterpret_cast<const double2*>(p);
   double2 a = q[0], b = q[1];

@@ -351,12 +351,15 @@ __device__ __forceinline__ void cell_body(const DevT<R>& d, VBlock vb, Gas<doubl
   __shared__ R s_qp[SL ? BLK * 4 : 1];
   __shared__ R s_cen[SL ? BLK * 2 : 1];
   __shared__ R s_t[SL && WITH_T ? BLK : 1];
+  __shared__ __align__(16) R s_rec[GRAD != G_NONE || LIMIT ? BLK / 64 : 1][32 * RW];
   const int base = xcd_block(vb.b, vb.n) * BLK;
-  const int c = base + threadIdx.x;
   const int cnt = min(BLK, d.noc - base);
+  // lanes past the last cell take it again and store nothing
+  const bool act = (int)threadIdx.x < cnt;
+  const int c = base + min((int)threadIdx.x, cnt - 1);
   R own[RW];
   R tc = R(0);
-  if (c < d.noc) {
+  {
     // the fields this kernel reads, from compact arrays (whole lines of
     // them, where the records would give a few values per line): the
     // primitives (which the last stage of a whole iteration refreshes), the
@@ -369,14 +372,12 @@ __device__ __forceinline__ void cell_body(const DevT<R>& d, VBlock vb, Gas<doubl
     tc = d.qTc[c];
   }
   if (SL) {
-    if (c < d.noc) {
-      stv<R, 4>(s_qp + threadIdx.x * 4, own + R_QP);
-      stv<R, 2>(s_cen + threadIdx.x * 2, own + R_CEN);
-      if (WITH_T) s_t[threadIdx.x] = tc;
-    }
+    stv<R, 4>(s_qp + threadIdx.x * 4, own + R_QP);
+    stv<R, 2>(s_cen + threadIdx.x * 2, own + R_CEN);
+    if (WITH_T) s_t[threadIdx.x] = tc;
     __syncthreads();
   }
-  if (c >= d.noc || d.err[0]) return;
+  if (d.err[0]) return;
   const int noc = d.noc;
   int info = ld_nt(d.cnf + c), nf = info & 0xff, nb = info >> 8;
   R cx = own[R_CEN], cy = own[R_CEN + 1];
@@ -511,7 +512,7 @@ __device__ __forceinline__ void cell_body(const DevT<R>& d, VBlock vb, Gas<doubl
     for (int k = 0; k < 8; ++k) own[R_G + k] = gr[k];
     if (WITH_T) {
       R t2[2] = {gr[8], gr[9]};
-      stv<R, 2>(d.gT + (size_t)c * 2, t2);
+      if (act) stv<R, 2>(d.gT + (size_t)c * 2, t2);
     }
   }
   if (LIMIT) {
@@ -538,9 +539,13 @@ __device__ __forceinline__ void cell_body(const DevT<R>& d, VBlock vb, Gas<doubl
   // and the gradient, for the stages' neighbour gathers
   static_assert(R_PHI == R_QP + 4 && R_G == R_PHI + 4, "record fields are adjacent");
   if (GRAD != G_NONE || LIMIT) {
-    stv<R, 16>(d.rec + (size_t)c * RW + R_QP, own + R_QP);
-    d.qT[c] = tc;
+#pragma unroll
+    for (int k = R_CEN + 2; k < RW; ++k) own[k] = R(0);
+    const int w = (int)threadIdx.x / 64;
+    store_records<R, RW, 32>(d.rec, base + w * 64, cnt - w * 64, own, s_rec[w]);
+    if (act) d.qT[c] = tc;
   }
+  if (!act) return;
   if (LIMIT) stv<R, 4>(d.phc + (size_t)c * 4, own + R_PHI);
   if (TSTEP) {
     double dt = cfl * d.cv[c] / la;

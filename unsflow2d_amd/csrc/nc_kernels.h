@@ -332,6 +332,9 @@ __global__ __launch_bounds__(BLK) void k_nc_grad_lim(DevNC d, NCFree g, int rev)
   // the same block
   __shared__ R s_qp[BLK * 4];
   __shared__ R s_xy[BLK * 2];
+  // (FP64: a block's LDS stays below what its registers allow)
+  constexpr int NR = sizeof(R) == 4 ? 64 : 32;
+  __shared__ __align__(16) R s_rec[BLK / 64][NR * W];
   // blocks past the vertices' form the boundary closures of this residual
   // evaluation (they read only primitives and coordinates, which this
   // kernel does not write)
@@ -342,20 +345,18 @@ __global__ __launch_bounds__(BLK) void k_nc_grad_lim(DevNC d, NCFree g, int rev)
     return;
   }
   const int base = xcd_block_dir(blockIdx.x, nvb, rev != 0) * BLK;
-  const int p = base + (int)threadIdx.x;
   const int cnt = min(BLK, d.nop - base);
+  // lanes past the last vertex take it again and store nothing
+  const int p = base + min((int)threadIdx.x, cnt - 1);
   const R* qps = NCRec<R>::qp(d);
   const R* xys = NCRec<R>::xy(d);
   const R* egg = NCRec<R>::gg(d);
   R q[4], xy[2];
-  if (p < d.nop) {
-    ldv<R, 4>(qps + (size_t)p * 4, q);
-    ldv<R, 2>(xys + (size_t)p * 2, xy);
-    stv<R, 4>(s_qp + threadIdx.x * 4, q);
-    stv<R, 2>(s_xy + threadIdx.x * 2, xy);
-  }
+  ldv<R, 4>(qps + (size_t)p * 4, q);
+  ldv<R, 2>(xys + (size_t)p * 2, xy);
+  stv<R, 4>(s_qp + threadIdx.x * 4, q);
+  stv<R, 2>(s_xy + threadIdx.x * 2, xy);
   __syncthreads();
-  if (p >= d.nop) return;
   auto nbr_qp = [&](int o, R* qo) {
     const unsigned l = (unsigned)(o - base);
     if (l < (unsigned)cnt) ldv<R, 4>(s_qp + l * 4, qo);
@@ -481,14 +482,19 @@ __global__ __launch_bounds__(BLK) void k_nc_grad_lim(DevNC d, NCFree g, int rev)
   // the record the residual gathers: primitives, limiter values and
   // gradient in one piece; and the limiter values' compact copy
   static_assert(R_PHI == R_QP + 4 && R_G == R_PHI + 4, "record fields are adjacent");
-  R o16[16];
-  ldv<R, 4>(s_qp + threadIdx.x * 4, o16);  // (read back: q need not stay live)
+  R o[W];
+  ldv<R, 4>(s_qp + threadIdx.x * 4, o);  // (read back: q need not stay live)
 #pragma unroll
-  for (int k = 0; k < 4; ++k) o16[4 + k] = phi[k];
+  for (int k = 0; k < 4; ++k) o[4 + k] = phi[k];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) o16[8 + k] = gr[k];
-  stv<R, 16>(NCRec<R>::rec(d) + (size_t)p * W + R_QP, o16);
-  stv<R, 4>(NCRec<R>::phc(d) + (size_t)p * 4, phi);
+  for (int k = 0; k < 8; ++k) o[8 + k] = gr[k];
+  static_assert(R_CEN == 16, "the coordinates follow");
+  ldv<R, 2>(s_xy + threadIdx.x * 2, o + R_CEN);
+#pragma unroll
+  for (int k = R_CEN + 2; k < W; ++k) o[k] = R(0);
+  const int w = (int)threadIdx.x / 64;
+  store_records<R, W, NR>(NCRec<R>::rec(d), base + w * 64, cnt - w * 64, o, s_rec[w]);
+  if ((int)threadIdx.x < cnt) stv<R, 4>(NCRec<R>::phc(d) + (size_t)p * 4, phi);
 }
 
 // Spectral radius of a dual face from the Roe average of its two states,
