@@ -77,7 +77,10 @@ __global__ __launch_bounds__(BLK) void k_face_lambda(DevT<R> d, Gas<double> g, d
 // CCFVM/main.F90:62-67 (con2prim of interior cells), qold = qc
 // (CCFVM/solution.F90:118-132), positivity (CCFVM/main.F90:384-411) and the
 // global range of the four primitives over all cells including ghosts
-// (CCFVM/limiter.F90:146-149), accumulated atomically.
+// (CCFVM/limiter.F90:146-149), accumulated atomically.  do_prim 2: whole
+// iterations, whose gradient pass stores the records' primitives (32 bytes of
+// each record here, the whole record there): 22 us instead of 32 on 640 000
+// cells.
 template <typename R>
 __device__ __forceinline__ void prim_body(const DevT<R>& d, VBlock vb, Gas<double> g, int do_prim,
                                           int do_old, int do_range) {
@@ -98,9 +101,11 @@ __device__ __forceinline__ void prim_body(const DevT<R>& d, VBlock vb, Gas<doubl
         con2prim(g, q, p);
 #pragma unroll
         for (int k = 0; k < 4; ++k) q4[k] = (R)p[k];
-        stv<R, 4>(d.rec + (size_t)c * RW + R_QP, q4);
+        if (do_prim == 1) {
+          stv<R, 4>(d.rec + (size_t)c * RW + R_QP, q4);
+          d.qT[c] = (R)p[4];
+        }
         stv<R, 4>(d.qpc + (size_t)c * 4, q4);
-        d.qT[c] = (R)p[4];
         d.qTc[c] = (R)p[4];
         // check_positivity (CCFVM/main.F90:384-411) runs after the
         // iteration's update on these start-of-iteration values; the
@@ -602,10 +607,14 @@ __global__ __launch_bounds__(BLK) void k_ggfc_face(DevT<R> d) {
   R a[PW], b[PW], qi[4], qo[4], ci2[2], co2[2];
   ldv<R, PW>(d.prec + (size_t)pp.x * PW, a);
   ldv<R, PW>(d.prec + (size_t)pp.y * PW, b);
-  ldv<R, 4>(d.rec + (size_t)ci * RW + R_QP, qi);
-  ldv<R, 4>(d.rec + (size_t)co * RW + R_QP, qo);
-  ldv<R, 2>(d.rec + (size_t)ci * RW + R_CEN, ci2);
-  ldv<R, 2>(d.rec + (size_t)co * RW + R_CEN, co2);
+  // (the inner cell is interior; whole lines of the compact arrays where the
+  // records would give a few values per line: 49 us instead of 64 on 960 000
+  // faces)
+  ldv<R, 4>(d.qpc + (size_t)ci * 4, qi);
+  if (co < d.noc) ldv<R, 4>(d.qpc + (size_t)co * 4, qo);
+  else ldv<R, 4>(d.rec + (size_t)co * RW + R_QP, qo);
+  ldv<R, 2>(d.cenc + (size_t)ci * 2, ci2);
+  ldv<R, 2>(d.cenc + (size_t)co * 2, co2);
   R pr[3][5];
   double x[3], y[3];
   R g1[10], g2[10];
@@ -616,14 +625,14 @@ __global__ __launch_bounds__(BLK) void k_ggfc_face(DevT<R> d) {
   x[2] = d.px[pp.y]; y[2] = d.py[pp.y];
   for (int k = 0; k < 5; ++k) { pr[0][k] = a[k]; pr[2][k] = b[k]; }
   for (int k = 0; k < 4; ++k) pr[1][k] = qo[k];
-  pr[1][4] = d.qT[co];
+  pr[1][4] = co < d.noc ? d.qTc[co] : d.qT[co];
   bool ok = gradtri(x, y, pr, g1, a1);
   // triangle (p1, p2, in)
   x[1] = d.px[pp.y]; y[1] = d.py[pp.y];
   x[2] = (double)ci2[0]; y[2] = (double)ci2[1];
   for (int k = 0; k < 5; ++k) { pr[0][k] = a[k]; pr[1][k] = b[k]; }
   for (int k = 0; k < 4; ++k) pr[2][k] = qi[k];
-  pr[2][4] = d.qT[ci];
+  pr[2][4] = d.qTc[ci];
   ok = gradtri(x, y, pr, g2, a2) && ok;
   if (!ok) { set_err(d, DERR_AREA, d.fref[f]); return; }
   R o[10];
@@ -883,7 +892,8 @@ __device__ __forceinline__ bool face_flux_ab(const Gas<R>& gr, const R* ra, cons
 template <typename R>
 __device__ __forceinline__ void stage_end(const DevT<R>& d, int c, int op, double ak, double bk,
                                           int write_res, const double* r) {
-  if (op == 0 || write_res) st4d_nt(d.res + (size_t)c * 4, r);
+  if (op == 2) st4d_nt(d.lower + (size_t)c * 4, r);
+  else if (op == 0 || write_res) st4d_nt(d.res + (size_t)c * 4, r);
   if (op == 1) {
     double dta = ld_nt(d.dta + c), o[4], q[4];
     ld4d_nt(d.qold + (size_t)c * 4, o);
@@ -974,18 +984,20 @@ __device__ __forceinline__ void rk3_reduce(const DevT<R>& d, int slot, int epi, 
 }
 
 // Residual stage over the block's cells (gather_residual), routine by
-// routine: store the residual (op 0), or apply the stage update of
-// CCFVM/main.F90:92-101 in place (op 1; no other cell reads this cell's
-// state during a stage).  rev: the XCDs walk their slices of blocks from the
+// routine: store the residual (op 0; op 2: in `lower`, for k_visc_stage), or
+// apply the stage update of CCFVM/main.F90:92-101 in place (op 1; no other
+// cell reads this cell's state during a stage).  list: the blocks to run (null:
+// all).  rev: the XCDs walk their slices of blocks from the
 // far end.  SL: the block's records are first copied to LDS, so the
 // neighbours inside the block (most of them, the cells being
 // Hilbert-ordered) are read from there instead of through L2.
 template <typename R, int FLUX, bool SL>
-__global__ __launch_bounds__(BLK) void k_stage(DevT<R> d, Gas<R> gr, int op, int rev, double ak,
-                                               double bk, int write_res) {
+__global__ __launch_bounds__(BLK) void k_stage(DevT<R> d, Gas<R> gr, int op, const int* list,
+                                               int rev, double ak, double bk, int write_res) {
   extern __shared__ double lds_raw[];
   R* srec = reinterpret_cast<R*>(lds_raw);  // [BLK][RW] when SL
-  const int base = xcd_block_dir(blockIdx.x, gridDim.x, rev != 0) * BLK;
+  const int b = xcd_block_dir(blockIdx.x, gridDim.x, rev != 0);
+  const int base = (list ? list[b] : b) * BLK;
   const int c = base + threadIdx.x;
   if (SL) {
     stage_block_recs(d, srec, base, min(BLK, d.noc - base));
@@ -1311,9 +1323,11 @@ __device__ __forceinline__ void blk_residual(const DevT<R>& d, int c, int info, 
 
 // k_stage with the block's fluxes evaluated once.
 template <typename R, int FLUX, bool SL>
-__global__ __launch_bounds__(BLK) void k_stage_blk(DevT<R> d, Gas<R> gr, int op, int rev,
-                                                   double ak, double bk, int write_res) {
-  const int b = xcd_block_dir(blockIdx.x, gridDim.x, rev != 0);
+__global__ __launch_bounds__(BLK) void k_stage_blk(DevT<R> d, Gas<R> gr, int op,
+                                                   const int* list, int rev, double ak,
+                                                   double bk, int write_res) {
+  const int i = xcd_block_dir(blockIdx.x, gridDim.x, rev != 0);
+  const int b = list ? list[i] : i;
   bool run;
   const R* fl = blk_fluxes<R, FLUX, SL>(d, b, gr, &run);
   const int c = b * BLK + threadIdx.x;
@@ -1405,32 +1419,28 @@ __global__ __launch_bounds__(BLK, 2) void k_rk3_all(DevT<R> d, Gas<R> gr, Gas<do
 // Sutherland viscosity of the interior cells from the current state,
 // CCFVM/viscous_flux.F90:20-22,127-139.
 template <typename R>
-__global__ __launch_bounds__(BLK) void k_visc_mul(DevT<R> d, Gas<double> g) {
-  int c = cell_index();
-  if (c >= d.noc || d.err[0]) return;
-  double q[4], p[5];
-  ld4d(d.qc + (size_t)c * 4, q);
+__device__ __forceinline__ R visc_mul(const Gas<double>& g, const double* q) {
+  double p[5];
   con2prim(g, q, p);
   double num = 1.0 + 300.0 / 110.4;
   double den = p[4] + 300.0 / 110.4;
-  d.cmul[c] = (R)((num / den) * pow(p[4], 1.5));
+  return (R)((num / den) * pow(p[4], 1.5));
+}
+template <typename R>
+__global__ __launch_bounds__(BLK) void k_visc_mul(DevT<R> d, Gas<double> g) {
+  int c = cell_index();
+  if (c >= d.noc || d.err[0]) return;
+  double q[4];
+  ld4d(d.qc + (size_t)c * 4, q);
+  d.cmul[c] = visc_mul<R>(g, q);
 }
 
-// The viscous flux of every face once (the two cells of an interior face
-// see the same face viscosity, velocities and gradients,
-// CCFVM/viscous_flux.F90:24-76): the flux times the face length into fvis
-// (the residual adds it at `out`, subtracts it at `in`), the face viscosity,
-// and for boundary faces the wall force terms.
+// The viscous flux of face f per unit of mu / rey and of length: components 0
+// (energy), 2 and 3 (momentum), CCFVM/viscous_flux.F90:24-76.
 template <typename R>
-__global__ __launch_bounds__(BLK) void k_visc_face(DevT<R> d, Gas<double> g, double rey,
-                                                   double m_inf, double* bfluxv) {
-  const int f = cell_index();
-  if (f >= d.nof || d.err[0]) return;
-  const int noc = d.noc, ci = d.fin[f], co = d.fout[f];
-  const double mu = co < noc ? 0.5 * ((double)d.cmul[ci] + (double)d.cmul[co]) : (double)d.cmul[ci];
-  R fr[Layout<R>::FW];
-  face_rec(d, f, fr);
-  const double nx = fr[F_NX], ny = fr[F_NY], area = fr[F_AREA];
+__device__ __forceinline__ void visc_coef(const DevT<R>& d, const Gas<double>& g, double m_inf,
+                                          int f, const R* fr, double* F) {
+  const double nx = fr[F_NX], ny = fr[F_NY];
   R fq[5];
   face_prims<R, 3>(d, f, fq);
   R fg[10];
@@ -1443,15 +1453,30 @@ __global__ __launch_bounds__(BLK) void k_visc_face(DevT<R> d, Gas<double> g, dou
   double tauyy = two_third * (two * vy - ux);
   double factor = (g.gamma - 1.0) * m_inf * m_inf * 0.72;
   double qx = -(tx / factor), qy = -(ty / factor);
-  double mr = mu / rey;
-  double F[4];
-  F[0] = mr * ((uvel * tauxx + vvel * tauxy - qx) * nx + (uvel * tauxy + vvel * tauyy - qy) * ny);
+  F[0] = (uvel * tauxx + vvel * tauxy - qx) * nx + (uvel * tauxy + vvel * tauyy - qy) * ny;
   F[1] = 0.0;
-  F[2] = mr * (tauxx * nx + tauxy * ny);
-  F[3] = mr * (tauxy * nx + tauyy * ny);
-  double o[4];
+  F[2] = tauxx * nx + tauxy * ny;
+  F[3] = tauxy * nx + tauyy * ny;
+}
+
+// The viscous flux of every face once (the two cells of an interior face
+// see the same face viscosity, velocities and gradients): the flux times the
+// face length into fvis (the residual adds it at `out`, subtracts it at
+// `in`), the face viscosity, and for boundary faces the wall force terms.
+template <typename R>
+__global__ __launch_bounds__(BLK) void k_visc_face(DevT<R> d, Gas<double> g, double rey,
+                                                   double m_inf, double* bfluxv) {
+  const int f = cell_index();
+  if (f >= d.nof || d.err[0]) return;
+  const int noc = d.noc, ci = d.fin[f], co = d.fout[f];
+  const double mu = co < noc ? 0.5 * ((double)d.cmul[ci] + (double)d.cmul[co]) : (double)d.cmul[ci];
+  R fr[Layout<R>::FW];
+  face_rec(d, f, fr);
+  const double area = fr[F_AREA], mr = mu / rey;
+  double F[4], o[4];
+  visc_coef<R>(d, g, m_inf, f, fr, F);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) o[i] = F[i] * area;
+  for (int i = 0; i < 4; ++i) o[i] = (i == 1 ? 0.0 : mr * F[i]) * area;
   st4d(d.fvis + (size_t)f * 4, o);
   d.fmu[f] = mu;
   if (co >= noc) {
@@ -1459,6 +1484,74 @@ __global__ __launch_bounds__(BLK) void k_visc_face(DevT<R> d, Gas<double> g, dou
     bfluxv[k] = -o[2];
     bfluxv[d.nbf + k] = -o[3];
   }
+}
+
+// Whole iterations with the diamond-path gradient: velocities and gradients
+// of a face are those of the iteration's start in all three stages, only the
+// viscosity follows the stage state.  Once per iteration the fluxes per unit
+// viscosity and length, with the length (fvis).
+template <typename R>
+__global__ __launch_bounds__(BLK) void k_visc_coef(DevT<R> d, Gas<double> g, double m_inf) {
+  const int f = cell_index();
+  if (f >= d.nof || d.err[0]) return;
+  R fr[Layout<R>::FW];
+  face_rec(d, f, fr);
+  double F[4];
+  visc_coef<R>(d, g, m_inf, f, fr, F);
+  F[1] = (double)fr[F_AREA];
+  st4d(d.fvis + (size_t)f * 4, F);
+}
+
+// A stage's residual of every cell: its inviscid residual, which the stage
+// pass left in `lower` (the interior one is the same in every stage), and the
+// viscous fluxes of its faces in ascending order, as k_visc_face and
+// k_visc_sum form them.  last: also the face viscosities (from the face's
+// `in` cell) and the wall force terms.  A face's flux is three products here,
+// so both its cells form it rather than one storing it for them.  On 640 000
+// cells 22 us a stage (and once 29 us for k_visc_coef), where k_visc_mul,
+// k_visc_face and k_visc_sum take 65 us.
+template <typename R>
+__global__ __launch_bounds__(BLK) void k_visc_stage(DevT<R> d, double rey, int last,
+                                                    double* bfluxv) {
+  const int c = cell_index();
+  if (c >= d.noc || d.err[0]) return;
+  const int noc = d.noc, nf = ld_nt(d.cnf + c) & 0xff;
+  int sf[MAXF], sn[MAXF];
+#pragma unroll
+  for (int s = 0; s < MAXF; ++s)
+    if (s < nf) {
+      sf[s] = ld_nt(d.sl_face + s * noc + c);
+      sn[s] = ld_nt(d.sl_nbr + s * noc + c);
+    }
+  const double own = (double)d.cmul[c];
+  double r[4];
+  ld4d(d.lower + (size_t)c * 4, r);
+#pragma unroll
+  for (int s = 0; s < MAXF; ++s) {
+    if (s >= nf) break;
+    const bool in_side = sn[s] >= 0;
+    const int n = in_side ? sn[s] : ~sn[s];
+    const double mu = n < noc ? 0.5 * (own + (double)d.cmul[n]) : own, mr = mu / rey;
+    double F[4], o[4];
+    ld4d(d.fvis + (size_t)sf[s] * 4, F);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (i == 1 ? 0.0 : mr * F[i]) * F[1];
+    if (in_side) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = r[i] - o[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = r[i] + o[i];
+    }
+    if (last && in_side) {
+      d.fmu[sf[s]] = mu;
+      if (n >= noc) {
+        bfluxv[n - noc] = -o[2];
+        bfluxv[d.nbf + n - noc] = -o[3];
+      }
+    }
+  }
+  st4d(d.res + (size_t)c * 4, r);
 }
 
 // The viscous fluxes summed into each cell's residual over its faces in
@@ -1496,13 +1589,14 @@ __global__ __launch_bounds__(BLK) void k_visc_sum(DevT<R> d) {
 // One Jacobi sweep of the central implicit residual smoothing,
 // CCFVM/ImpResiSmoothening.F90:27-44.
 // upd: also the stage update of CCFVM/main.F90:92-101 with the smoothed
-// residual (the last sweep), as k_rk_update does it.
+// residual (the last sweep), as k_rk_update does it; 2: and the viscosity of
+// the new state, for the next stage.  norm: and the block's partial of the
+// squared residual, as k_sumsq forms it.
 template <typename R>
-__global__ __launch_bounds__(BLK) void k_cirs(DevT<R> d, double eps, const double* src,
-                                              const double* old, double* dst, int upd,
-                                              double ak, double bk) {
-  int c = cell_index();
-  if (c >= d.noc || d.err[0]) return;
+__device__ __forceinline__ void cirs_cell(const DevT<R>& d, const Gas<double>& g, int c,
+                                          double eps, const double* src, const double* old,
+                                          double* dst, int upd, double ak, double bk,
+                                          double* out) {
   const int noc = d.noc;
   int info = d.cnf[c], nf = info & 0xff, nb = info >> 8;
   double it[4] = {0, 0, 0, 0};
@@ -1514,7 +1608,7 @@ __global__ __launch_bounds__(BLK) void k_cirs(DevT<R> d, double eps, const doubl
     for (int i = 0; i < 4; ++i) it[i] = it[i] + v[i];
   }
   double den = 1.0 / (1.0 + eps * (double)d.nc2c[c]);
-  double o[4], out[4];
+  double o[4];
   ld4d(old + (size_t)c * 4, o);
   for (int i = 0; i < 4; ++i) out[i] = (it[i] * eps + o[i]) * den;
   st4d(dst + (size_t)c * 4, out);
@@ -1524,7 +1618,24 @@ __global__ __launch_bounds__(BLK) void k_cirs(DevT<R> d, double eps, const doubl
     ld4d(d.qold + (size_t)c * 4, qo);
     for (int i = 0; i < 4; ++i) q[i] = rk_update1(ak, qo[i], bk, q[i], dta, out[i]);
     st4d(d.qc + (size_t)c * 4, q);
+    if (upd == 2) d.cmul[c] = visc_mul<R>(g, q);
   }
+}
+template <typename R>
+__global__ __launch_bounds__(BLK) void k_cirs(DevT<R> d, Gas<double> g, double eps,
+                                              const double* src, const double* old, double* dst,
+                                              int upd, double ak, double bk, int norm) {
+  __shared__ double sh[1][BLK];
+  const int c = cell_index();
+  double out[4] = {0.0, 0.0, 0.0, 0.0};
+  const bool run = !d.err[0];
+  if (run && c < d.noc) cirs_cell<R>(d, g, c, eps, src, old, dst, upd, ak, bk, out);
+  else if (norm && c < d.noc) ld4d(d.res + (size_t)c * 4, out);
+  if (!norm) return;
+  double sq = 0.0;
+  for (int i = 0; i < 4; ++i) sq = sq + out[i] * out[i];
+  block_reduce<1>(sh, &sq, OpAdd());
+  if (threadIdx.x == 0) d.part[blockIdx.x] = sq;
 }
 
 // Stage update alone, CCFVM/main.F90:92-101.
