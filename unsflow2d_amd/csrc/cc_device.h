@@ -89,9 +89,13 @@ struct DevT {
   const double *cv, *cov;    // noc (cov: ncell)
   const int* nc2c;
   const int* cref;           // storage cell -> reference cell number (ncell)
-  const int *v2c_ptr, *v2c;  // point storage order
+  // cells around a point and their pseudo-Laplacian weights in R, points in
+  // storage order: the first AVG_UNR slot-major, the others in tail lists
+  const int *v2n, *v2c;      // [nop] count; [AVG_UNR][nop]
+  const R* wt;               // [AVG_UNR][nop]
+  const int *v2t_ptr, *v2t;  // [nop] start of a point's tail; the tails
+  const R* wtt;
   const int* avg_w0;         // per block of BLK vertices: its lowest interior cell
-  const R* wt;                // pseudo-Laplacian weights per v2c entry, in R
   const double *px, *py;     // point storage order
   const int *fin, *fout;     // face sides (storage numbering of faces)
   const int* fref;           // storage face -> reference face number (error reports)

@@ -1072,7 +1072,26 @@ int build_dev(ufx_cc* x, DevT<R>& d, const Mesh& m, const std::vector<int>& sl_f
   UP(fref, x->ref_of_face);
   UP(r11, r11); UP(r12, r12); UP(r22, r22); UP(cv, cv); UP(cov, cov);
   UP(nc2c, nc2c); UP(cref, x->ref_of_sto);
-  UP(v2c_ptr, v2c_ptr); UP(v2c, v2c); UP(wt, wt); UP(px, px); UP(py, py); UP(avg_w0, avg_w0);
+  {
+    std::vector<int> v2n(nop), vs((size_t)AVG_UNR * nop, 0), v2t_ptr(nop), v2t;
+    std::vector<R> ws((size_t)AVG_UNR * nop, R(0)), wtt;
+    for (int p = 0; p < nop; ++p) {
+      v2n[p] = v2c_ptr[p + 1] - v2c_ptr[p];
+      v2t_ptr[p] = (int)v2t.size();
+      for (int k = 0; k < v2n[p]; ++k) {
+        const int j = v2c_ptr[p] + k;
+        if (k < AVG_UNR) {
+          vs[(size_t)k * nop + p] = v2c[j];
+          ws[(size_t)k * nop + p] = wt[j];
+        } else {
+          v2t.push_back(v2c[j]);
+          wtt.push_back(wt[j]);
+        }
+      }
+    }
+    UP(v2n, v2n); UP(v2c, vs); UP(wt, ws); UP(v2t_ptr, v2t_ptr); UP(v2t, v2t); UP(wtt, wtt);
+  }
+  UP(px, px); UP(py, py); UP(avg_w0, avg_w0);
   UP(fin, fin); UP(fout, fout); UP(lu_face, lu_face); UP(lu_cnt, lu_cnt);
   UP(rec, rec); UP(qc, qc);
   {
