@@ -349,7 +349,9 @@ enum { G_NONE = 0, G_LSQR = 1, G_GG = 2, G_GGFC = 3 };
 // wdt = 0 (whole RK3 iterations, whose stages read only dt/A): the
 // spectral radius and dt are not stored; the same pass with GRAD = G_NONE,
 // TSTEP forms them from the face radii when something reads them.
-template <typename R, int GRAD, bool WITH_T, bool LIMIT, bool TSTEP>
+// LAM: the face radii formed here too, each by both of its cells and stored by
+// its `in` cell (k_face_lambda's arithmetic, which is not contracted).
+template <typename R, int GRAD, bool WITH_T, bool LIMIT, bool TSTEP, bool LAM = false>
 __device__ __forceinline__ void cell_body(const DevT<R>& d, VBlock vb, Gas<double> g, double vll,
                                           double cfl, int wdt = 1) {
   constexpr int RW = Layout<R>::RW, FW = Layout<R>::FW;
@@ -427,13 +429,20 @@ __device__ __forceinline__ void cell_body(const DevT<R>& d, VBlock vb, Gas<doubl
       fcy[s] = fc[1];
     }
     R fq[5];
-    if (GRAD == G_GG || (LIMIT && bnd)) {
+    if (GRAD == G_GG || LAM || (LIMIT && bnd)) {
       if (GRAD == G_GG) face_prims<R, 5>(d, f, fq);
       else face_prims<R, 4>(d, f, fq);
     }
     // cell spectral radius: the face radii of k_face_lambda summed in
     // ascending face order, CCFVM/timestep.F90:171-173
-    if (TSTEP) la = la + d.fla[f];
+    if (TSTEP && LAM) {
+      if (GRAD != G_GG) ldv<R, 4>(d.fnl + (size_t)f * 4, fr);
+      const double l1 = face_lambda_val<R>(g, fq, fr, 0.0, 0.0);
+      la = la + l1;
+      if (act && in_side) d.fla[f] = l1;
+    } else if (TSTEP) {
+      la = la + d.fla[f];
+    }
     R nq[4];
     const unsigned l = (unsigned)(n - base);
     const bool loc = SL && l < (unsigned)cnt;
@@ -564,10 +573,10 @@ __device__ __forceinline__ void cell_body(const DevT<R>& d, VBlock vb, Gas<doubl
     d.dta[c] = dt / d.cv[c];
   }
 }
-template <typename R, int GRAD, bool WITH_T, bool LIMIT, bool TSTEP>
+template <typename R, int GRAD, bool WITH_T, bool LIMIT, bool TSTEP, bool LAM = false>
 __global__ __launch_bounds__(BLK) void k_cell(DevT<R> d, Gas<double> g, double vll, double cfl,
                                               int wdt) {
-  cell_body<R, GRAD, WITH_T, LIMIT, TSTEP>(d, hw_block(), g, vll, cfl, wdt);
+  cell_body<R, GRAD, WITH_T, LIMIT, TSTEP, LAM>(d, hw_block(), g, vll, cfl, wdt);
 }
 
 // ------------------------------------------------ diamond-path face gradient

@@ -209,6 +209,8 @@ constexpr size_t STAGE_LDS_MAX = 64 * 1024;
 // k_rk3_all: blocks of one launch at most, and its LDS beside the stage's
 constexpr int RK3_ALL_BLOCKS = 512;
 constexpr size_t RK3_ALL_LDS = 12 * 1024;
+// blocks of cells up to which k_cell forms the face radii itself
+constexpr int CELL_LAM_BLOCKS = 512;
 
 int launch_check() {
   hipError_t e = hipGetLastError();
@@ -380,10 +382,12 @@ int run_avg_range(ufx_cc* x, DevT<R>& d, int nparts) {
 
 // k_cell with the options of one call; with_t when the temperature gradient
 // has a consumer (the drop-in gradient routines always produce it); tstep:
-// with the time step from the face radii of a k_face_lambda pass.  (Summing
-// radii evaluated inside k_cell instead saves that pass but doubled the
-// prec gathers' HBM traffic, the vertex averages no longer staying in L2
-// beside k_cell's other streams: same time, 1.36 instead of 1.09 GB.)
+// with the time step from the face radii of a k_face_lambda pass, or from
+// radii that k_cell forms itself on meshes of up to CELL_LAM_BLOCKS blocks.
+// (The latter saves a launch: an iteration on 20 000 cells takes 2 us less of
+// 41, on 100 000 4 us of 55; on two million cells it doubled the prec
+// gathers' HBM traffic, the vertex averages no longer staying in L2 beside
+// k_cell's other streams: same time, 1.36 instead of 1.09 GB.)
 template <typename R, int GR>
 int run_cell_g(ufx_cc* x, DevT<R>& d, bool with_t, bool limit, bool tstep, double cfl,
                int wdt = 1) {
@@ -393,6 +397,13 @@ int run_cell_g(ufx_cc* x, DevT<R>& d, bool with_t, bool limit, bool tstep, doubl
     x->dtla_cfl = cfl;
   }
   int cat = GR != G_NONE ? UFX_K_GRAD : (tstep ? UFX_K_TSTEP : UFX_K_GRAD);
+  if (GR == G_LSQR || GR == G_GG) {
+    if (tstep && limit && !with_t && vll == 0.0 && x->nblk_cell <= CELL_LAM_BLOCKS) {
+      LAUNCH(x, cat, (k_cell<R, GR, false, true, true, GR == G_LSQR || GR == G_GG>),
+             x->nblk_cell, d, x->g, vll, cfl, wdt);
+      return launch_check();
+    }
+  }
   if (tstep) {
     LAUNCH(x, UFX_K_TSTEP, k_face_lambda<R>, x->nblk_face, d, x->g, vll);
     if (int rc = launch_check()) return rc;
