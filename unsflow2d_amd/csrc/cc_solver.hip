@@ -2097,16 +2097,18 @@ int batch_write(ufx_cc_batch* b) {
 // One inviscid RK3 iteration of every active case, as run_iteration does it
 // for one context (the first active case's options hold for all): the
 // primitive refresh only when `refresh` (the first iteration of a call), the
-// last stage refreshing them for the next iteration.
+// last stage refreshing them for the next iteration and the norm's launch
+// forming their range (not for an iteration after the call's last).
 template <typename R>
-int batch_iteration(ufx_cc_batch* b, ufx_cc* x0, int k, double cfl, int keep, bool refresh) {
+int batch_iteration(ufx_cc_batch* b, ufx_cc* x0, int k, double cfl, int keep, bool refresh,
+                    bool last) {
   const CaseDesc<R>* cs = (const CaseDesc<R>*)b->d_desc;
   const hipStream_t s = b->stream;
   auto M = [&](int t) { return (const int4*)(b->d_map + b->off[t]); };
   auto G = [&](int t) { return dim3((unsigned)b->cnt[t]); };
   const bool lim = x0->p.ilimit != 0;
   if (refresh) km_prim<R><<<G(T_ALL), BLK, 0, s>>>(cs, M(T_ALL), 1, 2, lim ? 1 : 0);
-  if (lim) km_range_final<R><<<G(T_CASE), BLK, 0, s>>>(cs, M(T_CASE), refresh ? 0 : 1);
+  if (lim && refresh) km_range_final<R><<<G(T_CASE), BLK, 0, s>>>(cs, M(T_CASE));
   km_avg_c2v<R, false><<<G(T_PT), BLK, 0, s>>>(cs, M(T_PT));
   km_face_lambda<R><<<G(T_FACE), BLK, 0, s>>>(cs, M(T_FACE));
 #define KMC(GR)                                                                            \
@@ -2139,7 +2141,7 @@ int batch_iteration(ufx_cc_batch* b, ufx_cc* x0, int k, double cfl, int keep, bo
     default: KMS(4); break;
   }
 #undef KMS
-  km_norm_final<R><<<G(T_CASE), BLK, 0, s>>>(cs, M(T_CASE), k);
+  km_norm_final<R><<<G(T_CASE), BLK, 0, s>>>(cs, M(T_CASE), k, lim && !last ? 1 : 0);
   return launch_check();
 }
 
@@ -2190,13 +2192,13 @@ int batch_iterate(ufx_cc_batch* b, int niter, double cfl) {
                      b->chunk.keep != keep || niter > b->chunk.n;
   if (!fresh && niter < b->chunk.n) {
     for (int k = 0; k < niter; ++k)
-      if (int rc = batch_iteration<R>(b, x0, k, cfl, keep, k == 0)) return rc;
+      if (int rc = batch_iteration<R>(b, x0, k, cfl, keep, k == 0, k == niter - 1)) return rc;
   } else {
     if (fresh) {
       HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
       int rc = 0;
       for (int k = 0; k < niter && !rc; ++k)
-        rc = batch_iteration<R>(b, x0, k, cfl, keep, k == 0);
+        rc = batch_iteration<R>(b, x0, k, cfl, keep, k == 0, k == niter - 1);
       Chunk c;
       hipError_t e = hipStreamEndCapture(b->stream, &c.graph);
       if (!rc && e == hipSuccess) e = hipGraphInstantiate(&c.exec, c.graph, nullptr, nullptr, 0);
