@@ -103,7 +103,7 @@ def kernel_name(category: str, precision: str, form: str) -> str:
         k, lds = STAGE_KERNELS[form]
         return f"ufx::{k}<{r},1,{lds}>"
     if category == "gradient":
-        return f"ufx::k_cell<{r},1,false,true,true>"
+        return f"ufx::k_cell<{r},1,false,true,true,false>"
     if category == "time_step":
         return f"ufx::k_face_lambda<{r}>"
     return f"ufx::k_avg_c2v_range<{r},false>"
@@ -377,9 +377,9 @@ def main_nc(args) -> int:
 
 
 # algorithmic HBM bytes per cell-stage of the second-order inviscid RK3
-# iteration (LSQ + limiter + Roe), the per-pass model of the cell-centred
-# path: 468.8 B in FP64, 296.7 B in the mixed form
-MODEL_BYTES_PER_CELL_STAGE = {"fp64": 468.8, "mixed": 296.7}
+# iteration (LSQ + limiter + Roe): a third of iteration_bytes, whose residual
+# pass serves the three stages
+MODEL_BYTES_PER_CELL_STAGE = {"fp64": 247.4, "mixed": 144.7}
 
 
 def sequential_baseline(cs, precision: str, maxiter: int, window: int) -> dict:

@@ -276,10 +276,13 @@ int ufx_cc_forces(ufx_cc* ctx, double* out, double* cp, double* cf);
  * iteration iter0+1+k (the host evaluates the reference's ramp).  hist, if
  * not NULL, receives the normalised residual of each iteration; that makes the
  * call synchronising.  Without hist no host synchronisation happens.
- * Inviscid RK3 iterations without residual smoothing keep the iteration's
- * start state in "qc" through the stages (the stage states live in a
- * separate buffer) instead of copying it to "qold": after them "qold" still
- * holds what the last save_old (or LU-SGS / viscous iteration) stored.
+ * Inviscid RK3 iterations without residual smoothing read the iteration's
+ * start state from "qc", which a cell's three stage updates overwrite once,
+ * instead of copying it to "qold": after them "qold" still holds what the
+ * last save_old (or LU-SGS / viscous iteration) stored.
+ * A stage's residual differs from the one before it only through the wall
+ * faces (and the viscosity of a laminar flow): whole iterations evaluate what
+ * no stage changes once.
  * They store no "la" / "dt" either: those of the last time step are formed
  * from the face radii when get, set, forces or LU-SGS read them (the same
  * values bit for bit). */
