@@ -91,6 +91,18 @@ struct Readback {
   }
 };
 
+// The context's device made current, the caller's put back at the end.
+struct DeviceGuard {
+  int was = -1;
+  explicit DeviceGuard(int device) {
+    if (hipGetDevice(&was) != hipSuccess || was == device || hipSetDevice(device) != hipSuccess)
+      was = -1;
+  }
+  ~DeviceGuard() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+};
+
 inline int read_failed(hipError_t e) {
   (void)hipGetLastError();
   set_error(std::string("read-back: ") + hipGetErrorString(e));
@@ -103,6 +115,7 @@ static int read_rows(Readback& rb, int device, hipStream_t stream, const double*
   constexpr size_t ROW = W * sizeof(double);
   const size_t bytes = n * ROW;
   if (n == 0) return UFX_OK;
+  const DeviceGuard guard(device);
   if (hipError_t e = rb.reserve(bytes)) return read_failed(e);
   auto gather = [&](size_t i0, size_t m, char* to) {
     const size_t th = W == 4 ? 2 * m : m;
