@@ -674,9 +674,9 @@ int run_lusgs(ufx_cc* x, DevT<R>& d) {
     // (triangles have at most three neighbours to a sweep)
 #define KSW(ME)                                                                                 \
   do {                                                                                          \
-    LAUNCH(x, UFX_K_OTHER, (k_sweep<CcSweep, ME, false, CC_SW_RING, 0>), 1, sc, x->sw, 0,       \
+    LAUNCH(x, UFX_K_OTHER, (k_sweep<CcSweep, ME, 0, CC_SW_RING, 0>), 1, sc, x->sw, 0,       \
            x->sw_npass[0], x->sw_nstep[0], d.qc, d.err);                                        \
-    LAUNCH(x, UFX_K_OTHER, (k_sweep<CcSweep, ME, false, CC_SW_RING, 1>), 1, sc, x->sw,          \
+    LAUNCH(x, UFX_K_OTHER, (k_sweep<CcSweep, ME, 0, CC_SW_RING, 1>), 1, sc, x->sw,          \
            x->sw_npass[0], x->sw_npass[1], x->sw_nstep[1], d.qc, d.err);                        \
   } while (0)
     if (x->sw_maxe <= 3) KSW(3);

@@ -50,6 +50,7 @@ struct ufx_nc {
   SweepSlot* d_slots = nullptr;             // packed sweep slots, forward then backward
   SweepDev sw{};                            // one-workgroup sweeps over the level order (sweep.h)
   int sw_npass[2] = {0, 0}, sw_nstep[2] = {0, 0};  // passes and steps of the forward and the backward sweep
+  bool sw_spill = false;                    // a vertex has more far neighbours than a pass fetches
   int nwall = 0;                            // wall edges (bc 1001)
   int* d_wedge = nullptr;                   // their stored edges, in ascending reference order
   std::vector<int> es, es_ref;              // storage slot of each reference edge, and back
@@ -281,10 +282,16 @@ int run_lusgs(ufx_nc* x, double cfl) {
     const NcSweep sc{x->g, x->d.dd};
     NLAUNCH(x, NK_LUSGS, k_sweep_prep<NcSweep>, nblk_of(2 * x->nop), sc, x->sw, x->d.res,
             x->d.qold, x->d.fla, (const int*)nullptr);
-    NLAUNCH(x, NK_LUSGS, (k_sweep<NcSweep, SW_ENTRIES, true, SW_RING, 0>), 1, sc, x->sw, 0,
-            x->sw_npass[0], x->sw_nstep[0], x->d.qc, (const int*)nullptr);
-    NLAUNCH(x, NK_LUSGS, (k_sweep<NcSweep, SW_ENTRIES, true, SW_RING, 1>), 1, sc, x->sw,
-            x->sw_npass[0], x->sw_npass[1], x->sw_nstep[1], x->d.qc, (const int*)nullptr);
+#define KSW(TAIL)                                                                               \
+  do {                                                                                          \
+    NLAUNCH(x, NK_LUSGS, (k_sweep<NcSweep, SW_ENTRIES, TAIL, SW_RING, 0>), 1, sc, x->sw, 0,     \
+            x->sw_npass[0], x->sw_nstep[0], x->d.qc, (const int*)nullptr);                      \
+    NLAUNCH(x, NK_LUSGS, (k_sweep<NcSweep, SW_ENTRIES, TAIL, SW_RING, 1>), 1, sc, x->sw,        \
+            x->sw_npass[0], x->sw_npass[1], x->sw_nstep[1], x->d.qc, (const int*)nullptr);      \
+  } while (0)
+    if (x->sw_spill) KSW(2);
+    else KSW(1);
+#undef KSW
     return launch_ok();
   }
   NLAUNCH(x, NK_LUSGS, k_nc_lusgs_diag, x->nblk, x->d);
@@ -793,6 +800,7 @@ int ufx_nc_create(const ufx_mesh* mesh, const ufx_nc_params* prm, ufx_nc** out) 
       SweepDev& w = x->sw;
       w.np = (int)np;
       w.node = x->lv_verts;
+      x->sw_spill = pl.spill;
       for (int dir = 0; dir < 2; ++dir) {
         x->sw_npass[dir] = pl.npass[dir];
         x->sw_nstep[dir] = pl.nstep[dir];

@@ -20,7 +20,8 @@
 //     in an LDS ring of the last SW_RING positions;
 //   - a neighbour further back (a few per cent of the reads) is fetched from
 //     its stored record passes ahead into a second LDS area, at a slot that
-//     the host has assigned: inside a pass every read is an LDS read;
+//     the host has assigned: inside a pass every read is an LDS read (but for
+//     nodes with more neighbours further back than a pass can fetch);
 //   - the four waves take the passes in turn: while one (or, in a wide level,
 //     several) updates its nodes, the others store the results of their last
 //     pass and issue the loads of their next ones, which would otherwise stand
@@ -46,32 +47,9 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-#include <vector>
+#include "sweep_plan.h"
 
 namespace ufx {
-
-constexpr int SW_WAVES = 4;      // one wave per SIMD: the loads ahead take its registers
-constexpr int SW_WIDTH = 64;     // nodes of a pass, lanes of a wave
-constexpr int SW_THREADS = SW_WAVES * SW_WIDTH;
-constexpr int SW_MAXE = 5;       // entries of a node that are loaded ahead
-constexpr int SW_REC = 9;        // doubles per LDS slot: dq (4), rho, u, v, p, E + p
-constexpr int SW_GREC = 10;      // doubles per stored record (the same, whole 16-byte loads)
-// LDS slots of a sweep with a ring of `ring`: the ring, the fetched records
-// of each wave, a record of zeros (what unused entries read); a multiple of
-// 64.  The LDS holds value i of slot s at [i][s]: neighbours of consecutive
-// nodes are mostly consecutive, and so are their banks.
-constexpr int sw_zero_slot(int ring) { return ring + SW_THREADS; }
-constexpr int sw_slots(int ring) { return (sw_zero_slot(ring) + 64) / 64 * 64; }
-// When a stored record may be read.  After its update of pass p (wave p mod
-// 4) a wave stores that pass's results, then loads the stream of its pass
-// p + 8 and the records that pass reads.  A wave's vector memory operations
-// complete in order, so its update of pass y, which waits for what it loaded
-// after pass y - 8, shows its stores of pass y - 8 done, and the barrier that
-// ends the step of pass y passes this on.  Records for pass p are loaded
-// after the step of pass p - 8: the stores of pass p - 16 and before are
-// done.  So a record that is fetched is at least SW_GAP passes old.
-constexpr int SW_GAP = 16;
 
 // Device side of a plan.  Positions: the forward sweep's nodes in its order,
 // then the backward sweep's; np = 2 nodes.  rows: the most entries of a node,
@@ -82,10 +60,10 @@ struct SweepDev {
   const int* far = nullptr;    // [passes][SW_WIDTH] position whose record the lane fetches, or -1
   const int4* head = nullptr;  // [np] the first five entries' LDS slots (16 bits each); then in z
                                // the entry count << 16 and the sign bit if the node's record is
-                               // fetched by some pass; in w where its result goes (forward: the
+                               // read from memory by some pass; in w where its result goes (forward: the
                                // node's place in the backward order; backward: the node)
-  const int* more = nullptr;   // [rows][np] LDS slot of every entry (those past the fifth are read
-                               // here)
+  const int* more = nullptr;   // [rows][np] LDS slot of every entry, or bit-inverted the place of
+                               // its stored record (those past the fifth are read here)
   const int2* pe = nullptr;    // [rows][np] (edge, neighbour) for the preparing pass
   const int* node = nullptr;   // [np] node of each position
   double2* ent = nullptr;      // [rows][S::NE][np] the entries' data
@@ -94,91 +72,6 @@ struct SweepDev {
   double* fwd = nullptr;       // [nodes][4] the forward sweep's dq in backward order
   double* rec = nullptr;       // [nodes + 1][SW_GREC] stored records (by position within the sweep)
 };
-
-// ------------------------------------------------------------------- plan
-// Host side: the passes and slots of both sweeps.  verts: the nodes of the
-// forward levels, then of the backward levels; off: offsets of the levels
-// (both sweeps, into verts); per position the entries [eptr[s], eptr[s + 1])
-// of nb, each a neighbour's position; out: where a position's result goes.
-struct SweepPlan {
-  std::vector<int4> pass, head;
-  std::vector<int> far, slot;
-  int npass[2] = {0, 0}, nstep[2] = {0, 0};  // of the forward and the backward sweep
-  int q = SW_MAXE;
-};
-
-inline SweepPlan sweep_plan(int n, const std::vector<int>& off_f, const std::vector<int>& off_b,
-                            const std::vector<size_t>& eptr, const std::vector<int>& nb,
-                            const std::vector<int>& out, int ring) {
-  SweepPlan p;
-  const size_t np = 2 * (size_t)n;
-  std::vector<int> cnt(np);
-  std::vector<char> fetched(np, 0);
-  for (size_t s = 0; s < np; ++s) {
-    cnt[s] = (int)(eptr[s + 1] - eptr[s]);
-    p.q = std::max(p.q, cnt[s]);
-  }
-  p.slot.assign((size_t)p.q * np, sw_zero_slot(ring));
-  for (int dir = 0; dir < 2; ++dir) {
-    const std::vector<int>& off = dir == 0 ? off_f : off_b;
-    const int base = dir == 0 ? 0 : n;  // ring slots count from the sweep's first position
-    const int at0 = (int)p.pass.size();
-    int step = -1;
-    for (size_t l = 0; l + 1 < off.size(); ++l) {
-      if (off[l + 1] > off[l]) ++step;
-      for (int b = off[l]; b < off[l + 1];) {
-        // as many nodes of the level as fit: at most SW_WIDTH, and at most
-        // SW_WIDTH reads of stored records.  The ring is short of what the
-        // passes of the same step write.
-        const int at = (int)p.pass.size(), most = std::min(off[l + 1] - b, SW_WIDTH);
-        const int lim = b + SW_THREADS - ring;
-        // a wave's passes are in different steps
-        if (at - at0 >= SW_WAVES) step = std::max(step, p.pass[at - SW_WAVES].z + 1);
-        p.far.resize((size_t)(at + 1) * SW_WIDTH, -1);
-        int* far = &p.far[(size_t)at * SW_WIDTH];
-        int cnt_far = 0, m = 0, mc = 0;
-        for (; m < most; ++m) {
-          const size_t s = (size_t)b + m;
-          int need = 0;
-          for (size_t j = eptr[s]; j < eptr[s + 1]; ++j) need += nb[j] < lim;
-          if (cnt_far + need > SW_WIDTH && m > 0) break;
-          for (size_t j = eptr[s]; j < eptr[s + 1]; ++j) {
-            const int o = nb[j];
-            int sl;
-            if (o >= lim) {
-              sl = (o - base) % ring;
-            } else {
-              sl = ring + (at - at0) % SW_WAVES * SW_WIDTH + cnt_far;
-              far[cnt_far++] = o - base;
-              fetched[o] = 1;
-            }
-            p.slot[(j - eptr[s]) * np + s] = sl;
-          }
-          mc = std::max(mc, cnt[s]);
-        }
-        p.pass.push_back(make_int4(b, m, step, mc));
-        b += m;
-      }
-    }
-    // whole groups of eight passes (two to each wave; the kernel's loop has
-    // no exit inside one): the last pass again, whose inputs are still in place
-    while (((int)p.pass.size() - at0) % (2 * SW_WAVES) != 0) {
-      int4 w = p.pass.back();
-      w.z = ++step;
-      p.pass.push_back(w);
-      p.far.resize(p.pass.size() * SW_WIDTH, -1);
-    }
-    p.npass[dir] = (int)p.pass.size() - at0;
-    p.nstep[dir] = step + 1;
-  }
-  p.head.resize(np);
-  for (size_t s = 0; s < np; ++s) {
-    auto sl = [&](int k) { return p.slot[(size_t)k * np + s]; };
-    p.head[s] = make_int4(sl(0) | sl(1) << 16, sl(2) | sl(3) << 16,
-                          sl(4) | cnt[s] << 16 | (fetched[s] ? (int)0x80000000 : 0), out[s]);
-  }
-  return p;
-}
 
 // ---------------------------------------------------------------- kernels
 // What a sweep reads in its order: per position the node's residual (negated),
@@ -288,8 +181,10 @@ __device__ __forceinline__ void sweep_div4(const double* a, double b, double y, 
 
 // One sweep over npass passes (a multiple of 8) in nstep steps.  S: the
 // solver's terms (term), update (update) and primitives (prims).  ME entries
-// of a node are loaded ahead; TAIL: some have more.
-template <typename S, int ME, bool TAIL, int RING, int DIR>
+// of a node are loaded ahead; TAIL 1: some have more; 2: and some of those are
+// read from their stored records (SweepPlan::spill; a kernel of its own: the
+// branch costs the others half a per cent).
+template <typename S, int ME, int TAIL, int RING, int DIR>
 __global__ __launch_bounds__(SW_THREADS, 1) void k_sweep(S sc, SweepDev d, int pass0, int npass,
                                                          int nstep, double* qc, const int* err) {
   static_assert(ME <= SW_MAXE && RING >= SW_THREADS + SW_GAP * SW_WIDTH,
@@ -345,13 +240,25 @@ __global__ __launch_bounds__(SW_THREADS, 1) void k_sweep(S sc, SweepDev d, int p
         const int h = k < 2 ? sg.head.x : k < 4 ? sg.head.y : sg.head.z;
         add((k & 1) ? (int)((unsigned)h >> 16) : h & 0xffff, sg.e[k]);
       }
-    if (TAIL)
+    if (TAIL > 0)
       for (int k = ME; k < ((sg.head.z >> 16) & 0x7fff); ++k) {
         const size_t np = (size_t)d.np, s = (size_t)sg.b + ll;
         double2 e[NE];
 #pragma unroll
         for (int i = 0; i < NE; ++i) e[i] = d.ent[((size_t)k * NE + i) * np + s];
-        add(d.more[(size_t)k * np + s], e);
+        const int sl = d.more[(size_t)k * np + s];
+        if (TAIL == 1 || sl >= 0) {
+          add(sl, e);
+        } else {
+          const double2* rec = recs + 5 * (size_t)~sl;
+          double nb[SW_REC + 1];
+#pragma unroll
+          for (int i = 0; i < 5; ++i) {
+            nb[2 * i] = rec[i].x;
+            nb[2 * i + 1] = rec[i].y;
+          }
+          sc.term(nb, e, cres);
+        }
       }
     const double res[4] = {sg.r01.x, sg.r01.y, sg.r23.x, sg.r23.y};
     const double pd[4] = {sg.p01.x, sg.p01.y, sg.p23.x, sg.p23.y};
