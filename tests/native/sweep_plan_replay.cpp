@@ -3,7 +3,7 @@
 // rests on.  Prints one line per sweep; exit status 1 on the first violation.
 //
 //   sweep_plan_replay RING grid NI NJ | cells NI NJ | shuffled NI NJ SEED |
-//                     layers WIDTH COUNT BACK | hub N WHERE
+//                     layers WIDTH COUNT BACK | hub N WHERE | limits
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -236,6 +236,24 @@ static int replay(const Graph& g, int ring) {
   return 0;
 }
 
+// no plan past what the kernel's 32-bit offsets and 15-bit counts hold
+static int limits(int ring) {
+  const std::vector<int> none(1, 0);
+  if (sweep_plan((1 << 26) + 1, none, none, {}, none, none, ring).npass[0])
+    return bad("no plan of more than 2^27 positions");
+  // node 0 last in the backward sweep, with 2^15 neighbours; one level a sweep is enough here
+  const int n = (1 << 15) + 1;
+  std::vector<int> f(2), b(3), nb(2 * (size_t)(n - 1), 0), out(2 * (size_t)n, 0);
+  f = {0, 1, n};
+  b = {n, 2 * n - 1, 2 * n};
+  std::vector<size_t> eptr(1, 0);
+  for (int s = 0; s < 2 * n; ++s) eptr.push_back(eptr.back() + (s == 0 || (s >= n && s < 2 * n - 1) ? 0 : s < n ? 1 : n - 1));
+  for (int i = 0; i < n - 1; ++i) nb[(size_t)n - 1 + i] = n + i;
+  if (sweep_plan(n, f, b, eptr, nb, out, ring).npass[0])
+    return bad("no plan of a node with 2^15 neighbours");
+  return 0;
+}
+
 int main(int argc, char** argv) {
   if (argc < 3) return 2;
   const int ring = std::atoi(argv[1]);
@@ -245,6 +263,7 @@ int main(int argc, char** argv) {
   if (kind == "cells") return replay(cells(a(3), a(4)), ring);
   if (kind == "shuffled") return replay(renumbered(grid(a(3), a(4)), (unsigned)a(5)), ring);
   if (kind == "layers") return replay(layers(a(3), a(4), a(5)), ring);
+  if (kind == "limits") return limits(ring);
   if (kind == "hub") return replay(hub(a(3), a(4)), ring);
   return 2;
 }

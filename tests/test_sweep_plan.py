@@ -67,3 +67,10 @@ def test_nodes_of_any_number_of_neighbours(replay, n, where):
     spilt = max(int(m) for m in re.findall(r"(\d+) from memory", out))
     if where != "middle":
         assert spilt == max(0, n - 1 - 1280 - 64)
+
+
+def test_no_plan_past_the_kernel_limits(replay):
+    """More positions than the kernel's 32-bit offsets reach (2^27), or more
+    neighbours of a node than its 15-bit count holds: the caller sweeps by
+    level launches instead."""
+    replay(_ring(*RINGS["nc"]), "limits")

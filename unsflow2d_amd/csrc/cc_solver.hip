@@ -1434,10 +1434,10 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
     // A step takes 0.7 us, a level's launch 7 us: the launches are faster
     // only where a level is more than ten steps (a level is two or three
     // steps on a channel of two million triangles).  They also remain where
-    // the plan does not fit the memory or its 32-bit offsets.
+    // the plan does not fit the memory or the kernel's offsets.
     const size_t steps = (size_t)pl.nstep[0] + pl.nstep[1];
     const size_t levels = x->lv_fwd_off.size() + x->lv_bwd_off.size() - 2;
-    if (steps <= 10 * levels + 16 && need < mem_free / 2 && np <= ((size_t)1 << 27)) {
+    if (pl.npass[0] > 0 && steps <= 10 * levels + 16 && need < mem_free / 2) {
       std::vector<int2> pe(rows * np, make_int2(0, 0));
       std::vector<double2> ent(rows * CcSweep::NE * np, make_double2(0.0, 0.0));
       // the face geometry as the face records hold it

@@ -761,6 +761,7 @@ int ufx_nc_create(const ufx_mesh* mesh, const ufx_nc_params* prm, ufx_nc** out) 
     // the one-workgroup sweeps over the level order: per position the swept
     // neighbours in edge order, their passes and LDS slots, and position-major
     // the edge geometry (unused slots: zeros, never read)
+    bool planned = false;
     {
       const size_t np = verts.size();
       std::vector<int> pos(np);  // position of each vertex in each sweep
@@ -784,51 +785,54 @@ int ufx_nc_create(const ufx_mesh* mesh, const ufx_nc_params* prm, ufx_nc** out) 
         out[s] = dir == 0 ? pos[(size_t)nop + p] - nop : p;
       }
       const SweepPlan pl = sweep_plan(nop, cf, cb, eptr, nb, out, SW_RING);
-      const size_t nq = (size_t)pl.q;
-      std::vector<int2> pe(nq * np, make_int2(0, 0));
-      std::vector<double2> ent(nq * 4 * np, make_double2(0.0, 0.0));
-      for (size_t s = 0; s < np; ++s)
-        for (size_t j = eptr[s]; j < eptr[s + 1]; ++j) {
-          const size_t k = j - eptr[s];
-          const bool inv = eo_all[j].x < 0;
-          const int e = inv ? ~eo_all[j].x : eo_all[j].x;
-          pe[k * np + s] = make_int2(es[e], eo_all[j].y);
-          ent[k * 4 * np + s] = inv ? make_double2(-m.fnx[e], -m.fny[e])
-                                    : make_double2(m.fnx[e], m.fny[e]);
-          ent[(k * 4 + 1) * np + s] = make_double2(m.farea[e], 0.0);
+      planned = pl.npass[0] > 0;
+      if (planned) {
+        const size_t nq = (size_t)pl.q;
+        std::vector<int2> pe(nq * np, make_int2(0, 0));
+        std::vector<double2> ent(nq * 4 * np, make_double2(0.0, 0.0));
+        for (size_t s = 0; s < np; ++s)
+          for (size_t j = eptr[s]; j < eptr[s + 1]; ++j) {
+            const size_t k = j - eptr[s];
+            const bool inv = eo_all[j].x < 0;
+            const int e = inv ? ~eo_all[j].x : eo_all[j].x;
+            pe[k * np + s] = make_int2(es[e], eo_all[j].y);
+            ent[k * 4 * np + s] = inv ? make_double2(-m.fnx[e], -m.fny[e])
+                                      : make_double2(m.fnx[e], m.fny[e]);
+            ent[(k * 4 + 1) * np + s] = make_double2(m.farea[e], 0.0);
+          }
+        SweepDev& w = x->sw;
+        w.np = (int)np;
+        w.node = x->lv_verts;
+        x->sw_spill = pl.spill;
+        for (int dir = 0; dir < 2; ++dir) {
+          x->sw_npass[dir] = pl.npass[dir];
+          x->sw_nstep[dir] = pl.nstep[dir];
         }
-      SweepDev& w = x->sw;
-      w.np = (int)np;
-      w.node = x->lv_verts;
-      x->sw_spill = pl.spill;
-      for (int dir = 0; dir < 2; ++dir) {
-        x->sw_npass[dir] = pl.npass[dir];
-        x->sw_nstep[dir] = pl.nstep[dir];
+        if (!rc) rc = nc_upload(x, &w.pass, pl.pass);
+        if (!rc) rc = nc_upload(x, &w.far, pl.far);
+        if (!rc) rc = nc_upload(x, &w.head, pl.head);
+        if (!rc) rc = nc_upload(x, &w.more, pl.slot);
+        if (!rc) rc = nc_upload(x, &w.pe, pe);
+        if (!rc) rc = nc_upload(x, &w.ent, ent);
+        if (!rc) rc = nc_alloc(x, &w.own, 4 * np);
+        if (!rc) rc = nc_alloc(x, &w.diag, np);
+        if (!rc) rc = nc_alloc(x, &w.fwd, 4 * (size_t)nop);
+        if (!rc) rc = nc_alloc(x, &w.rec, (size_t)SW_GREC * (nop + 1));
       }
-      if (!rc) rc = nc_upload(x, &w.pass, pl.pass);
-      if (!rc) rc = nc_upload(x, &w.far, pl.far);
-      if (!rc) rc = nc_upload(x, &w.head, pl.head);
-      if (!rc) rc = nc_upload(x, &w.more, pl.slot);
-      if (!rc) rc = nc_upload(x, &w.pe, pe);
-      if (!rc) rc = nc_upload(x, &w.ent, ent);
-      if (!rc) rc = nc_alloc(x, &w.own, 4 * np);
-      if (!rc) rc = nc_alloc(x, &w.diag, np);
-      if (!rc) rc = nc_alloc(x, &w.fwd, 4 * (size_t)nop);
-      if (!rc) rc = nc_alloc(x, &w.rec, (size_t)SW_GREC * (nop + 1));
     }
     if (rc) { ufx_nc_destroy(x); return rc; }
     // sweep form: one workgroup over the level-ordered data (default,
-    // UFX_NC_SWEEP=stream), a replayed graph of the level launches (graph),
-    // the level launches themselves (levels), one workgroup walking the
-    // packed slots (single; needs at most SWQ swept neighbours per vertex),
-    // or one cooperative launch of several workgroups (grid)
+    // UFX_NC_SWEEP=stream; without a plan the level launches), a replayed
+    // graph of the level launches (graph), the level launches themselves
+    // (levels), one workgroup walking the packed slots (single; needs at most
+    // SWQ swept neighbours per vertex), or one cooperative launch of several
+    // workgroups (grid)
     const char* env = std::getenv("UFX_NC_SWEEP");
-    x->sweep_mode = 4;
+    x->sweep_mode = planned ? 4 : 1;
     if (env && std::strcmp(env, "graph") == 0) x->sweep_mode = 0;
     if (env && std::strcmp(env, "levels") == 0) x->sweep_mode = 1;
     if (env && std::strcmp(env, "single") == 0 && fits) x->sweep_mode = 2;
     if (env && std::strcmp(env, "grid") == 0) x->sweep_mode = 3;
-    if (env && std::strcmp(env, "stream") == 0) x->sweep_mode = 4;
     if (const char* w = std::getenv("UFX_NC_SWEEP_WGS")) x->grid_wgs = std::max(1, std::min(64, std::atoi(w)));
   }
   {

@@ -125,7 +125,7 @@ __device__ __forceinline__ T sweep_ld(const T* base, unsigned bytes) {
 template <typename S, int ME, int DIR>
 __device__ __forceinline__ void sweep_load(const SweepDev& d, int l, SweepStage<ME, S::NE>& st) {
   const size_t np = (size_t)d.np;
-  // uniform bases and 32-bit lane offsets (a plan has at most 2^27 positions)
+  // uniform bases and 32-bit lane offsets (a plan has at most SW_MAX_POS positions)
   const unsigned s = (unsigned)(st.b + min(l, st.n - 1));
   st.head = sweep_ld(d.head, s * 16);
 #pragma unroll

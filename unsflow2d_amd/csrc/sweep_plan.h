@@ -34,6 +34,11 @@ constexpr int sw_slots(int ring) { return (sw_zero_slot(ring) + 64) / 64 * 64; }
 // that a pass reads from memory itself could be 8 passes younger.)
 constexpr int SW_GAP = 16;
 
+// What the kernel's offsets hold: 32 bits for 32 bytes a node (both sweeps'
+// positions), and 15 bits of a position's head for its count of entries.
+constexpr size_t SW_MAX_POS = (size_t)1 << 27;
+constexpr size_t SW_MAX_CNT = (1 << 15) - 1;
+
 // Host side: the passes and slots of both sweeps.  verts: the nodes of the
 // forward levels, then of the backward levels; off: offsets of the levels
 // (both sweeps, into verts); per position the entries [eptr[s], eptr[s + 1])
@@ -42,6 +47,8 @@ constexpr int SW_GAP = 16;
 // a mesh, of any number) reads those that have no slot from their stored
 // records, slot[] being the bit-inverted place there; never one of its first
 // SW_MAXE entries, which take at most as many of its pass's SW_WIDTH slots.
+// No passes: the nodes or a node's entries are more than the kernel takes,
+// and the caller sweeps by level launches.
 struct SweepPlan {
   std::vector<int4> pass, head;
   std::vector<int> far, slot;
@@ -55,6 +62,9 @@ inline SweepPlan sweep_plan(int n, const std::vector<int>& off_f, const std::vec
                             const std::vector<int>& out, int ring) {
   SweepPlan p;
   const size_t np = 2 * (size_t)n;
+  if (np > SW_MAX_POS) return p;
+  for (size_t s = 0; s < np; ++s)
+    if (eptr[s + 1] - eptr[s] > SW_MAX_CNT) return p;
   std::vector<int> cnt(np);
   std::vector<char> fetched(np, 0);
   for (size_t s = 0; s < np; ++s) {
