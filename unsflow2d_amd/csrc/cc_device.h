@@ -132,7 +132,11 @@ struct DevT {
   int* err;                  // [0] code, [1] and [2] lowest 1-based reference cell with
                              // rho <= 0 or p <= 0 among the primitives the next iteration
                              // starts from ([1], noted by the last stage) and the current
-                             // one started from ([2]), [3] lowest failing face key (set_err)
+                             // one started from ([2]), [3] lowest failing face key (set_err),
+                             // [4] no error was pending before the stages of a whole iteration
+                             // (set by the norm before it or by its primitive refresh): what
+                             // they go by, the same in every wave whatever is reported in [0]
+                             // meanwhile
   double* lower;             // LU-SGS work [noc][4]
   double* upper;
 };

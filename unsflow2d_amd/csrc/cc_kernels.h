@@ -90,6 +90,8 @@ __device__ __forceinline__ void prim_body(const DevT<R>& d, VBlock vb, Gas<doubl
   double mx[4], mn[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) { mx[k] = -INFINITY; mn[k] = INFINITY; }
+  // (the RK3 stages that follow run)
+  if (do_old == 2 && vb.b == 0 && threadIdx.x == 0) d.err[4] = d.err[0] == 0;
   if (c < d.ncell && !d.err[0]) {
     R q4[4];
     if (c < d.noc && (do_prim || do_old)) {
@@ -646,7 +648,11 @@ __global__ __launch_bounds__(BLK) void k_ggfc_face(DevT<R> d) {
   for (int k = 0; k < 4; ++k) pr[2][k] = qi[k];
   pr[2][4] = d.qTc[ci];
   ok = gradtri(x, y, pr, g2, a2) && ok;
-  if (!ok) { set_err(d, DERR_AREA, d.fref[f]); return; }
+  if (!ok) {
+    set_err(d, DERR_AREA, d.fref[f]);
+    d.err[4] = 0;
+    return;
+  }
   R o[10];
   R A1 = (R)a1, A2 = (R)a2;
 #pragma unroll
@@ -1084,7 +1090,7 @@ __device__ __forceinline__ void rk3_body(const DevT<R>& d, VBlock vb, const Gas<
     stage_block_recs(d, srec, base, min(BLK, d.noc - base));
     __syncthreads();
   }
-  const int info = c < d.noc && !d.err[0] ? d.cnf[c] : -1;
+  const int info = c < d.noc && d.err[4] ? d.cnf[c] : -1;
   const bool have = info >= 0 && (info >> 8) == 0;
   // the cells with boundary faces: their interior fluxes for k_rk3_bcell in
   // the mixed form (FP64: that kernel evaluates them)
@@ -1122,7 +1128,11 @@ __global__ __launch_bounds__(BLK) void k_rk3(DevT<R> d, Gas<R> gr, Gas<double> g
 // stage updates, one lane per cell.  Interior and farfield fluxes do not
 // change over the stages; a wall's is evaluated in each.  A wall face failing
 // in a later stage counts after every failure of the earlier ones (the key
-// gets the stage in front, see set_err).
+// gets the stage in front, see set_err).  A Roe average that fails in this
+// very iteration, here or in the other cells, stops nothing of it: the waves
+// of a block take a cell together and must agree, and the reference's first
+// failing face may be a boundary face (looped first) when an interior one has
+// already been met.
 constexpr int BC_CELLS = BLK / MAXF;
 template <typename R, int FLUX>
 __device__ __forceinline__ void rk3_bcells(const DevT<R>& d, int t0, int t1, const Gas<R>& gr,
@@ -1137,7 +1147,7 @@ __device__ __forceinline__ void rk3_bcells(const DevT<R>& d, int t0, int t1, con
 #pragma unroll 1
   for (; t0 < t1; t0 += BC_CELLS) {
   const int t = t0 + l;
-  const bool run = t < t1 && !d.err[0];
+  const bool run = t < t1 && d.err[4];
   const int tc = min(t, t1 - 1), c = d.bc_cell[tc];
   const int4 tab = d.bc_tab[(size_t)s * d.nbc + tc];
   const int nf = tab.w & 0xff, ni = nf - (tab.w >> 8), f = tab.y;
@@ -1245,8 +1255,9 @@ __global__ __launch_bounds__(BLK) void k_rk3_bcell(DevT<R> d, int slot0, Gas<R> 
 // list has at most 2 BLK faces, the fluxes are held in registers until every
 // thread is done with the records and then written over them, so the block
 // needs no more LDS than its records.  Returns the flux list; *run: no error
-// was pending when the block started (uniform over the block).
-template <typename R, int FLUX, bool SL>
+// was pending when the block started, or with WHOLE when the iteration's
+// stages started (uniform over the block).
+template <typename R, int FLUX, bool SL, bool WHOLE>
 __device__ __forceinline__ const R* blk_fluxes(const DevT<R>& d, int b, const Gas<R>& gr,
                                                bool* run) {
   constexpr int RW = Layout<R>::RW, FW = Layout<R>::FW;
@@ -1254,7 +1265,7 @@ __device__ __forceinline__ const R* blk_fluxes(const DevT<R>& d, int b, const Ga
   R* srec = reinterpret_cast<R*>(lds_raw);
   R* fl = srec + (SL ? BLK * RW : 0);
   __shared__ int s_err;
-  if (threadIdx.x == 0) s_err = d.err[0];
+  if (threadIdx.x == 0) s_err = WHOLE ? d.err[4] == 0 : d.err[0];
   const int base = b * BLK;
   if (SL) stage_block_recs(d, srec, base, min(BLK, d.noc - base));
   __syncthreads();
@@ -1341,7 +1352,7 @@ __global__ __launch_bounds__(BLK) void k_stage_blk(DevT<R> d, Gas<R> gr, int op,
   const int i = xcd_block_dir(blockIdx.x, gridDim.x, rev != 0);
   const int b = list ? list[i] : i;
   bool run;
-  const R* fl = blk_fluxes<R, FLUX, SL>(d, b, gr, &run);
+  const R* fl = blk_fluxes<R, FLUX, SL, false>(d, b, gr, &run);
   const int c = b * BLK + threadIdx.x;
   if (!run || c >= d.noc) return;
   double r[4];
@@ -1356,7 +1367,7 @@ __device__ __forceinline__ void rk3_blk_body(const DevT<R>& d, VBlock vb, const 
                                              int epi, Rk3Acc& acc) {
   const int b = xcd_block_dir(vb.b, vb.n, rev != 0);
   bool run;
-  const R* fl = blk_fluxes<R, FLUX, SL>(d, b, gr, &run);
+  const R* fl = blk_fluxes<R, FLUX, SL, true>(d, b, gr, &run);
   const int c = b * BLK + threadIdx.x;
   const int info = run && c < d.noc ? ld_nt(d.cnf + c) : -1;
   const bool have = info >= 0 && (info >> 8) == 0;
@@ -1741,6 +1752,7 @@ __device__ __forceinline__ void norm_final_body(const DevT<R>& d, VBlock vb, int
       d.err[2] = d.err[1];
       d.err[1] = INT_MAX;
     }
+    d.err[4] = d.err[0] == 0;
     double fres = sqrt(s / d.noc / 4);
     d.scal[SC_NORM] = fres;
     if (first) d.scal[SC_FRES1] = fres;

@@ -1116,10 +1116,10 @@ int build_dev(ufx_cc* x, DevT<R>& d, const Mesh& m, const std::vector<int>& sl_f
   AL(bflux, 2 * (size_t)std::max(1, nbf)); AL(bres, 4 * (size_t)std::max(1, nbf));
   const size_t nparts = (size_t)std::max(x->nblk_all, x->nblk_cell + x->nblk_bc);
   AL(part, nparts); AL(rpart, nparts * 8);
-  AL(scal, SC_NSCAL); AL(range, 8); AL(err, 4); AL(lower, 4 * (size_t)noc); AL(upper, 4 * (size_t)noc);
+  AL(scal, SC_NSCAL); AL(range, 8); AL(err, 5); AL(lower, 4 * (size_t)noc); AL(upper, 4 * (size_t)noc);
 #undef UP
 #undef AL
-  int init[4] = {0, INT_MAX, INT_MAX, INT_MAX};
+  int init[5] = {0, INT_MAX, INT_MAX, INT_MAX, 0};
   HIPCHK(hipMemcpyAsync(d.err, init, sizeof(init), hipMemcpyHostToDevice, x->stream));
   unsigned long long rg[8] = {0, 0, 0, 0, ~0ULL, ~0ULL, ~0ULL, ~0ULL};
   HIPCHK(hipMemcpyAsync(d.range, rg, sizeof(rg), hipMemcpyHostToDevice, x->stream));
