@@ -389,7 +389,15 @@ __device__ __forceinline__ void cell_body(const DevT<R>& d, VBlock vb, Gas<doubl
     if (WITH_T) s_t[threadIdx.x] = tc;
     __syncthreads();
   }
-  if (d.err[0]) return;
+  if (d.err[0]) {
+    // (the diamond-path gradient stops after the primitives were refreshed:
+    // the record shows them as the reference's qp does)
+    if (GRAD == G_GGFC && act) {
+      stv<R, 4>(d.rec + (size_t)c * RW + R_QP, own + R_QP);
+      d.qT[c] = tc;
+    }
+    return;
+  }
   const int noc = d.noc;
   int info = ld_nt(d.cnf + c), nf = info & 0xff, nb = info >> 8;
   R cx = own[R_CEN], cy = own[R_CEN + 1];
