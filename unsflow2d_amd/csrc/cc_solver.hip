@@ -1385,6 +1385,9 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
   int rc = p.precision == UFX_PREC_FP64
                ? build_dev(x, x->d64, m, sl_face, sl_nbr, cnf, lu_face, lu_cnt, sl)
                : build_dev(x, x->d32, m, sl_face, sl_nbr, cnf, lu_face, lu_cnt, sl);
+  SweepPlan plan;  // its arrays go to the device last, below
+  std::vector<int2> sw_pe;
+  std::vector<double2> sw_ent;
   if (p.timemode == UFX_TIME_LUSGS && p.lusgs_order == UFX_LUSGS_REFERENCE) {
     // inside a level the order is free; cells of equal neighbour counts
     // together let a wave skip the entries that none of its cells has
@@ -1419,27 +1422,20 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
       eptr[s2 + 1] = eo_all.size();
       out[s2] = dir == 0 ? pos[(size_t)noc + it] - noc : it;
     }
-    const SweepPlan pl = sweep_plan(noc, x->lv_fwd_off, x->lv_bwd_off, eptr, nb, out, CC_SW_RING);
+    plan = sweep_plan(noc, x->lv_fwd_off, x->lv_bwd_off, eptr, nb, out, CC_SW_RING);
     for (size_t s2 = 0; s2 < np; ++s2)
       x->sw_maxe = std::max(x->sw_maxe, (int)(eptr[s2 + 1] - eptr[s2]));
-    const size_t rows = std::max(x->sw_maxe, 3);  // entry rows that the sweeps load
-    const size_t need = np * (rows * (16 * CcSweep::NE + 8) + 16 + 64 + 16) +
-                        (size_t)noc * (32 + 8 * SW_GREC) +
-                        pl.pass.size() * (16 + 4 * SW_WIDTH);
-    size_t mem_free = 0, mem_all = 0;
-    if (hipMemGetInfo(&mem_free, &mem_all) != hipSuccess) {
-      (void)hipGetLastError();
-      mem_free = 0;
-    }
     // A step takes 0.7 us, a level's launch 7 us: the launches are faster
     // only where a level is more than ten steps (a level is two or three
     // steps on a channel of two million triangles).  They also remain where
-    // the plan does not fit the memory or the kernel's offsets.
-    const size_t steps = (size_t)pl.nstep[0] + pl.nstep[1];
+    // the plan is past the kernel's offsets.  The mesh alone decides: the two
+    // forms differ in their last bits.
+    const size_t steps = (size_t)plan.nstep[0] + plan.nstep[1];
     const size_t levels = x->lv_fwd_off.size() + x->lv_bwd_off.size() - 2;
-    if (pl.npass[0] > 0 && steps <= 10 * levels + 16 && need < mem_free / 2) {
-      std::vector<int2> pe(rows * np, make_int2(0, 0));
-      std::vector<double2> ent(rows * CcSweep::NE * np, make_double2(0.0, 0.0));
+    if (plan.npass[0] > 0 && steps <= 10 * levels + 16) {
+      const size_t rows = std::max(x->sw_maxe, 3);  // entry rows that the sweeps load
+      sw_pe.assign(rows * np, make_int2(0, 0));
+      sw_ent.assign(rows * CcSweep::NE * np, make_double2(0.0, 0.0));
       // the face geometry as the face records hold it
       auto in_r = [&](double v) { return p.precision == UFX_PREC_FP64 ? v : (double)(float)v; };
       for (size_t s2 = 0; s2 < np; ++s2)
@@ -1448,31 +1444,17 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
           const bool inv = eo_all[j].x < 0;
           const int f = inv ? ~eo_all[j].x : eo_all[j].x;
           const double nx = in_r(m.fnx[f]), ny = in_r(m.fny[f]);
-          pe[k * np + s2] = make_int2(x->face_of_ref[f], eo_all[j].y);
-          ent[k * CcSweep::NE * np + s2] = inv ? make_double2(-nx, -ny) : make_double2(nx, ny);
-          ent[(k * CcSweep::NE + 1) * np + s2] = make_double2(in_r(m.farea[f]), 0.0);
+          sw_pe[k * np + s2] = make_int2(x->face_of_ref[f], eo_all[j].y);
+          sw_ent[k * CcSweep::NE * np + s2] = inv ? make_double2(-nx, -ny) : make_double2(nx, ny);
+          sw_ent[(k * CcSweep::NE + 1) * np + s2] = make_double2(in_r(m.farea[f]), 0.0);
         }
-      SweepDev& w = x->sw;
-      w.np = (int)np;
-      if (!rc) rc = dupload(x, &w.pass, pl.pass);
-      if (!rc) rc = dupload(x, &w.far, pl.far);
-      if (!rc) rc = dupload(x, &w.head, pl.head);
-      if (!rc) rc = dupload(x, &w.pe, pe);
-      if (!rc) rc = dupload(x, &w.ent, ent);
-      if (!rc) rc = dalloc(x, &w.own, 4 * np);
-      if (!rc) rc = dalloc(x, &w.diag, np);
-      if (!rc) rc = dalloc(x, &w.fwd, 4 * (size_t)noc);
-      if (!rc) rc = dalloc(x, &w.rec, (size_t)SW_GREC * (noc + 1));
-      for (int dir = 0; !rc && dir < 2; ++dir) {
-        x->sw_npass[dir] = pl.npass[dir];
-        x->sw_nstep[dir] = pl.nstep[dir];
-      }
+    } else {
+      plan = SweepPlan();
     }
   }
   if (!rc) rc = dupload(x, &x->d_sto, x->sto_of_ref);
   (void)x->rb.reserve((size_t)m.ncell() * 32);
   if (!rc) rc = dupload(x, &x->lv_cells, lv_cells);
-  x->sw.node = x->lv_cells;
   if (!rc && p.timemode == UFX_TIME_LUSGS && p.lusgs_order == UFX_LUSGS_MULTICOLOUR) {
     // colours of the interior cells (reference numbering) -> storage order;
     // each colour's cells in ascending storage order (compact blocks)
@@ -1499,6 +1481,34 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
   if (rc) {
     ufx_cc_destroy(x);
     return rc;
+  }
+  // the sweep's plan last: a context that fits the memory without it (560
+  // bytes a cell) sweeps by level launches
+  if (plan.npass[0] > 0) {
+    const size_t before = x->allocs.size(), np = 2 * (size_t)noc;
+    SweepDev& w = x->sw;
+    w.np = (int)np;
+    w.node = x->lv_cells;
+    int rs = dupload(x, &w.pass, plan.pass);
+    if (!rs) rs = dupload(x, &w.far, plan.far);
+    if (!rs) rs = dupload(x, &w.head, plan.head);
+    if (!rs) rs = dupload(x, &w.pe, sw_pe);
+    if (!rs) rs = dupload(x, &w.ent, sw_ent);
+    if (!rs) rs = dalloc(x, &w.own, 4 * np);
+    if (!rs) rs = dalloc(x, &w.diag, np);
+    if (!rs) rs = dalloc(x, &w.fwd, 4 * (size_t)noc);
+    if (!rs) rs = dalloc(x, &w.rec, (size_t)SW_GREC * (noc + 1));
+    if (hipStreamSynchronize(x->stream) != hipSuccess) rs = UFX_ERR_HIP;
+    for (int dir = 0; !rs && dir < 2; ++dir) {
+      x->sw_npass[dir] = plan.npass[dir];
+      x->sw_nstep[dir] = plan.nstep[dir];
+    }
+    if (rs) {
+      (void)hipGetLastError();
+      for (size_t i = before; i < x->allocs.size(); ++i) (void)hipFree(x->allocs[i]);
+      x->allocs.resize(before);
+      w = SweepDev{};
+    }
   }
   for (int k = 0; k < m.nbf; ++k)
     if (m.fbc[m.nfi + k] == WALL) x->wall_k.push_back(k);
