@@ -132,11 +132,18 @@ static int replay(const Graph& g, int ring) {
   }
   const SweepPlan p = sweep_plan(n, off[0], off[1], eptr, nb, out, ring);
   const size_t np = 2 * (size_t)n;
+  auto slot = [&](int k, int s) {
+    if (k >= SW_MAXE) return p.more[(size_t)(k - SW_MAXE) * np + s];
+    const int4 h = p.head[s];
+    const int w = k < 2 ? h.x : k < 4 ? h.y : h.z & 0xffff;
+    return k % 2 ? (int)((unsigned)w >> 16) : w & 0xffff;
+  };
   if (!p.npass[0] || !p.npass[1]) return bad("a plan");
   if (p.far.size() != p.pass.size() * SW_WIDTH) return bad("far size", p.far.size());
   if (sw_slots(ring) > 65536) return bad("slots fit 16 bits");
   for (int dir = 0; dir < 2; ++dir) {
     const int base = dir * n, p0 = dir == 0 ? 0 : p.npass[0], npass = p.npass[dir];
+    if (sweep_least_steps(off[dir]) > (size_t)p.nstep[dir]) return bad("least steps", dir);
     if (npass % (2 * SW_WAVES)) return bad("whole groups of passes", npass);
     std::vector<int> pass_of(n, -1), lev_of(n);
     for (size_t l = 0; l + 1 < off[dir].size(); ++l)
@@ -185,14 +192,9 @@ static int replay(const Graph& g, int ring) {
           if (h.w != out[s]) return bad("place of the result", s);
           for (int k = 0; k < cnt; ++k) {
             const int o = nb[eptr[s] + k], po = pass_of[o - base];
-            const int sl = p.slot[(size_t)k * np + s];
+            const int sl = slot(k, s);
             reads += i < real;
             if (po >= i || p.pass[p0 + po].z >= step) return bad("dependency", s, o);
-            if (k < SW_MAXE) {
-              const int hw = k < 2 ? h.x : k < 4 ? h.y : h.z & 0xffff;
-              const int hs = k % 2 ? (int)((unsigned)hw >> 16) : hw & 0xffff;
-              if (sl != hs) return bad("slot in the head", s, k);
-            }
             if (sl >= sw_slots(ring)) return bad("slot in the LDS", s, k, sl);
             if (sl >= 0 && sl < ring) {
               if (tag[sl] != o) return bad("ring slot holds the neighbour", s, o, tag[sl]);
@@ -216,7 +218,7 @@ static int replay(const Graph& g, int ring) {
             }
           }
           for (int k = cnt; k < p.q; ++k)
-            if (p.slot[(size_t)k * np + s] != sw_zero_slot(ring)) return bad("unused entry", s, k);
+            if (slot(k, s) != sw_zero_slot(ring)) return bad("unused entry", s, k);
         }
         if (mc != w.w) return bad("most entries", i, mc, w.w);
         for (int l = 0; l < SW_WIDTH; ++l) {

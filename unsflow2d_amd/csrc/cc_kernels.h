@@ -1949,6 +1949,27 @@ struct CcSweep {
   }
 };
 
+// The entries' geometry, from the face records (set-up): the normal outward
+// of the entry's cell, the face length.  (Formed on the host, the rows of two
+// million cells were 768 MB to fill and to copy.)
+template <typename R>
+__global__ __launch_bounds__(BLK) void k_sweep_geom(DevT<R> d, SweepDev w) {
+  const int s = cell_index();
+  if (s >= w.np) return;
+  const size_t np = (size_t)w.np;
+  const int node = w.node[s], cnt = (w.head[s].z >> 16) & 0x7fff;
+  for (int k = 0; k < cnt; ++k) {
+    const int f = w.pe[(size_t)k * np + s].x;
+    R fr[Layout<R>::FW];
+    face_rec(d, f, fr);
+    const double nx = fr[F_NX], ny = fr[F_NY];
+    const bool in = d.fin[f] == node;
+    double2* en = w.ent + (size_t)k * CcSweep::NE * np + s;
+    en[0] = in ? make_double2(nx, ny) : make_double2(-nx, -ny);
+    en[np] = make_double2(fr[F_AREA], 0.0);
+  }
+}
+
 // qc = qold + upper, CCFVM/lusgs.F90:314-318.
 template <typename R>
 __global__ __launch_bounds__(BLK) void k_lusgs_final(DevT<R> d) {

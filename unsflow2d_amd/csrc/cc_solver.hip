@@ -1271,12 +1271,15 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
     int f = m.c2f[m.c2f_ptr[c] + j];
     return m.fout[f] == c ? m.fin[f] : m.fout[f];
   };
+  const bool ref_lusgs =
+      prm->timemode == UFX_TIME_LUSGS && prm->lusgs_order == UFX_LUSGS_REFERENCE;
   int nlf = 0, nlb = 0;
+  std::vector<int> nlo(noc, 0), nhi(noc, 0);  // neighbours swept before a cell, both sweeps
   for (int c = 0; c < noc; ++c) {
     int l = 0;
     for (int j = 0; j < m.c2f_ptr[c + 1] - m.c2f_ptr[c]; ++j) {
       int o = nbr_of(c, j);
-      if (o < c && o >= 0) l = std::max(l, lvf[o] + 1);
+      if (o < c && o >= 0) { l = std::max(l, lvf[o] + 1); ++nlo[c]; }
     }
     lvf[c] = l;
     nlf = std::max(nlf, l + 1);
@@ -1285,27 +1288,35 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
     int l = 0;
     for (int j = 0; j < m.c2f_ptr[c + 1] - m.c2f_ptr[c]; ++j) {
       int o = nbr_of(c, j);
-      if (o > c && o < noc) l = std::max(l, lvb[o] + 1);
+      if (o > c && o < noc) { l = std::max(l, lvb[o] + 1); ++nhi[c]; }
     }
     lvb[c] = l;
     nlb = std::max(nlb, l + 1);
   }
-  std::vector<int> lv_cells(2 * (size_t)noc);  // storage indices, by level
-  {
-    std::vector<int> cnt(nlf + 1, 0);
-    for (int c = 0; c < noc; ++c) cnt[lvf[c] + 1]++;
-    for (int l = 0; l < nlf; ++l) cnt[l + 1] += cnt[l];
-    x->lv_fwd_off = cnt;
-    std::vector<int> pos(cnt.begin(), cnt.end() - 1);
-    for (int c = 0; c < noc; ++c) lv_cells[pos[lvf[c]]++] = sto[c];
-    std::vector<int> cb(nlb + 1, 0);
-    for (int c = 0; c < noc; ++c) cb[lvb[c] + 1]++;
-    for (int l = 0; l < nlb; ++l) cb[l + 1] += cb[l];
-    for (int l = 0; l <= nlb; ++l) cb[l] += noc;
-    x->lv_bwd_off = cb;
-    std::vector<int> pb(cb.begin(), cb.end() - 1);
-    for (int c = noc - 1; c >= 0; --c) lv_cells[pb[lvb[c]]++] = sto[c];
-  }
+  // storage indices by level, forward levels then backward, and the cells'
+  // places.  Inside a level the order is free: for the one-workgroup sweep,
+  // cells of equal neighbour counts together (most first) let a wave skip the
+  // entries that none of its cells has.
+  std::vector<int> lv_cells(2 * (size_t)noc), pos_f(noc), pos_b(noc);
+  auto by_level = [&](int nl, const std::vector<int>& lev, const std::vector<int>& cnt, bool fwd,
+                      std::vector<int>& off, std::vector<int>& pos) {
+    constexpr int B = MAXF + 1;
+    auto key = [&](int c) { return lev[c] * B + (ref_lusgs ? MAXF - cnt[c] : 0); };
+    const int base = fwd ? 0 : noc;
+    std::vector<int> at((size_t)nl * B + 1, 0);
+    for (int c = 0; c < noc; ++c) at[key(c) + 1]++;
+    at[0] = base;
+    for (size_t i = 0; i + 1 < at.size(); ++i) at[i + 1] += at[i];
+    off.resize(nl + 1);
+    for (int l = 0; l <= nl; ++l) off[l] = at[(size_t)l * B];
+    for (int i = 0; i < noc; ++i) {
+      const int c = fwd ? i : noc - 1 - i;
+      pos[c] = at[key(c)]++;
+      lv_cells[pos[c]] = sto[c];
+    }
+  };
+  by_level(nlf, lvf, nlo, true, x->lv_fwd_off, pos_f);
+  by_level(nlb, lvb, nhi, false, x->lv_bwd_off, pos_b);
   hipError_t e = hipGetDevice(&x->device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -1387,70 +1398,42 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
                : build_dev(x, x->d32, m, sl_face, sl_nbr, cnf, lu_face, lu_cnt, sl);
   SweepPlan plan;  // its arrays go to the device last, below
   std::vector<int2> sw_pe;
-  std::vector<double2> sw_ent;
-  if (p.timemode == UFX_TIME_LUSGS && p.lusgs_order == UFX_LUSGS_REFERENCE) {
-    // inside a level the order is free; cells of equal neighbour counts
-    // together let a wave skip the entries that none of its cells has
-    std::vector<int> nlo(noc, 0), nhi(noc, 0);
-    for (int c = 0; c < noc; ++c)
-      for (int j = 0; j < m.c2f_ptr[c + 1] - m.c2f_ptr[c]; ++j) {
-        const int o = nbr_of(c, j);
-        if (o < c) ++nlo[sto[c]];
-        else if (o < noc) ++nhi[sto[c]];
-      }
-    auto sort_levels = [&](const std::vector<int>& off, const std::vector<int>& cnt) {
-      for (size_t l = 0; l + 1 < off.size(); ++l)
-        std::stable_sort(lv_cells.begin() + off[l], lv_cells.begin() + off[l + 1],
-                         [&](int a, int b) { return cnt[a] > cnt[b]; });
-    };
-    sort_levels(x->lv_fwd_off, nlo);
-    sort_levels(x->lv_bwd_off, nhi);
+  // A step takes 0.7 us, a level's launch 7 us: the launches are faster only
+  // where a level is more than ten steps (a level is two or three steps on a
+  // channel of two million triangles).  They also remain where the plan is
+  // past the kernel's offsets.  The mesh alone decides: the two forms differ
+  // in their last bits.
+  const size_t most_steps = 10 * (x->lv_fwd_off.size() + x->lv_bwd_off.size() - 2) + 16;
+  if (ref_lusgs &&
+      sweep_least_steps(x->lv_fwd_off) + sweep_least_steps(x->lv_bwd_off) <= most_steps) {
+    // (cell by cell, whose neighbours are near in number: by position, the
+    // lists of two million cells took twice the time)
     const size_t np = 2 * (size_t)noc;
-    std::vector<int> pos(np), out(np), nb;
-    for (size_t s2 = 0; s2 < np; ++s2) pos[(s2 < (size_t)noc ? 0 : noc) + lv_cells[s2]] = (int)s2;
+    std::vector<int> out(np);
     std::vector<size_t> eptr(np + 1, 0);
-    std::vector<int2> eo_all;  // (reference face, bit-inverted when the cell is its `out`; neighbour)
-    for (size_t s2 = 0; s2 < np; ++s2) {
-      const int it = lv_cells[s2], c = x->ref_of_sto[it], dir = s2 < (size_t)noc ? 0 : 1;
-      for (int j = 0; j < m.c2f_ptr[c + 1] - m.c2f_ptr[c]; ++j) {
-        const int f = m.c2f[m.c2f_ptr[c] + j], o = nbr_of(c, j);
-        if (dir == 0 ? o < c : (o > c && o < noc)) {
-          eo_all.push_back(make_int2(m.fout[f] == c ? ~f : f, sto[o]));
-          nb.push_back(pos[(size_t)dir * noc + sto[o]]);
-        }
+    for (int c = 0; c < noc; ++c) {
+      eptr[(size_t)pos_f[c] + 1] = nlo[c];
+      eptr[(size_t)pos_b[c] + 1] = nhi[c];
+      x->sw_maxe = std::max({x->sw_maxe, nlo[c], nhi[c]});
+      out[pos_f[c]] = pos_b[c] - noc;
+      out[pos_b[c]] = sto[c];
+    }
+    for (size_t s2 = 0; s2 < np; ++s2) eptr[s2 + 1] += eptr[s2];
+    std::vector<int> nb(eptr[np]);
+    sw_pe.assign((size_t)std::max(x->sw_maxe, 3) * np, make_int2(0, 0));  // the rows that are loaded
+    for (int c = 0; c < noc; ++c) {
+      int kf = 0, kb = 0;
+      for (int j = m.c2f_ptr[c]; j < m.c2f_ptr[c + 1]; ++j) {
+        const int f = m.c2f[j], o = m.fout[f] == c ? m.fin[f] : m.fout[f];
+        if (o >= noc) continue;
+        const bool fwd = o < c;
+        const size_t at = fwd ? pos_f[c] : pos_b[c], k = fwd ? kf++ : kb++;
+        sw_pe[k * np + at] = make_int2(x->face_of_ref[f], sto[o]);
+        nb[eptr[at] + k] = fwd ? pos_f[o] : pos_b[o];
       }
-      eptr[s2 + 1] = eo_all.size();
-      out[s2] = dir == 0 ? pos[(size_t)noc + it] - noc : it;
     }
     plan = sweep_plan(noc, x->lv_fwd_off, x->lv_bwd_off, eptr, nb, out, CC_SW_RING);
-    for (size_t s2 = 0; s2 < np; ++s2)
-      x->sw_maxe = std::max(x->sw_maxe, (int)(eptr[s2 + 1] - eptr[s2]));
-    // A step takes 0.7 us, a level's launch 7 us: the launches are faster
-    // only where a level is more than ten steps (a level is two or three
-    // steps on a channel of two million triangles).  They also remain where
-    // the plan is past the kernel's offsets.  The mesh alone decides: the two
-    // forms differ in their last bits.
-    const size_t steps = (size_t)plan.nstep[0] + plan.nstep[1];
-    const size_t levels = x->lv_fwd_off.size() + x->lv_bwd_off.size() - 2;
-    if (plan.npass[0] > 0 && steps <= 10 * levels + 16) {
-      const size_t rows = std::max(x->sw_maxe, 3);  // entry rows that the sweeps load
-      sw_pe.assign(rows * np, make_int2(0, 0));
-      sw_ent.assign(rows * CcSweep::NE * np, make_double2(0.0, 0.0));
-      // the face geometry as the face records hold it
-      auto in_r = [&](double v) { return p.precision == UFX_PREC_FP64 ? v : (double)(float)v; };
-      for (size_t s2 = 0; s2 < np; ++s2)
-        for (size_t j = eptr[s2]; j < eptr[s2 + 1]; ++j) {
-          const size_t k = j - eptr[s2];
-          const bool inv = eo_all[j].x < 0;
-          const int f = inv ? ~eo_all[j].x : eo_all[j].x;
-          const double nx = in_r(m.fnx[f]), ny = in_r(m.fny[f]);
-          sw_pe[k * np + s2] = make_int2(x->face_of_ref[f], eo_all[j].y);
-          sw_ent[k * CcSweep::NE * np + s2] = inv ? make_double2(-nx, -ny) : make_double2(nx, ny);
-          sw_ent[(k * CcSweep::NE + 1) * np + s2] = make_double2(in_r(m.farea[f]), 0.0);
-        }
-    } else {
-      plan = SweepPlan();
-    }
+    if ((size_t)plan.nstep[0] + plan.nstep[1] > most_steps) plan = SweepPlan();
   }
   if (!rc) rc = dupload(x, &x->d_sto, x->sto_of_ref);
   (void)x->rb.reserve((size_t)m.ncell() * 32);
@@ -1493,7 +1476,13 @@ int ufx_cc_create(const ufx_mesh* mesh, const ufx_cc_params* prm, ufx_cc** out) 
     if (!rs) rs = dupload(x, &w.far, plan.far);
     if (!rs) rs = dupload(x, &w.head, plan.head);
     if (!rs) rs = dupload(x, &w.pe, sw_pe);
-    if (!rs) rs = dupload(x, &w.ent, sw_ent);
+    if (!rs) rs = dalloc(x, &w.ent, CcSweep::NE * sw_pe.size());  // (zeros)
+    if (!rs)
+      rs = with_dev(x, [&](auto& d) {
+        using R = typename std::remove_reference_t<decltype(d)>::Real;
+        LAUNCH(x, UFX_K_OTHER, k_sweep_geom<R>, nblocks((int)np), d, w);
+        return launch_check();
+      });
     if (!rs) rs = dalloc(x, &w.own, 4 * np);
     if (!rs) rs = dalloc(x, &w.diag, np);
     if (!rs) rs = dalloc(x, &w.fwd, 4 * (size_t)noc);

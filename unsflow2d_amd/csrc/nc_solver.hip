@@ -811,7 +811,7 @@ int ufx_nc_create(const ufx_mesh* mesh, const ufx_nc_params* prm, ufx_nc** out) 
         if (!rc) rc = nc_upload(x, &w.pass, pl.pass);
         if (!rc) rc = nc_upload(x, &w.far, pl.far);
         if (!rc) rc = nc_upload(x, &w.head, pl.head);
-        if (!rc) rc = nc_upload(x, &w.more, pl.slot);
+        if (!rc) rc = nc_upload(x, &w.more, pl.more);
         if (!rc) rc = nc_upload(x, &w.pe, pe);
         if (!rc) rc = nc_upload(x, &w.ent, ent);
         if (!rc) rc = nc_alloc(x, &w.own, 4 * np);

@@ -62,8 +62,8 @@ struct SweepDev {
                                // the entry count << 16 and the sign bit if the node's record is
                                // read from memory by some pass; in w where its result goes (forward: the
                                // node's place in the backward order; backward: the node)
-  const int* more = nullptr;   // [rows][np] LDS slot of every entry, or bit-inverted the place of
-                               // its stored record (those past the fifth are read here)
+  const int* more = nullptr;   // [rows - 5][np] LDS slot of each entry past the fifth, or
+                               // bit-inverted the place of its stored record
   const int2* pe = nullptr;    // [rows][np] (edge, neighbour) for the preparing pass
   const int* node = nullptr;   // [np] node of each position
   double2* ent = nullptr;      // [rows][S::NE][np] the entries' data
@@ -187,7 +187,7 @@ __device__ __forceinline__ void sweep_div4(const double* a, double b, double y, 
 template <typename S, int ME, int TAIL, int RING, int DIR>
 __global__ __launch_bounds__(SW_THREADS, 1) void k_sweep(S sc, SweepDev d, int pass0, int npass,
                                                          int nstep, double* qc, const int* err) {
-  static_assert(ME <= SW_MAXE && RING >= SW_THREADS + SW_GAP * SW_WIDTH,
+  static_assert((TAIL ? ME == SW_MAXE : ME <= SW_MAXE) && RING >= SW_THREADS + SW_GAP * SW_WIDTH,
                 "records out of the ring are SW_GAP passes old");
   constexpr int NE = S::NE, NS = sw_slots(RING);
   __shared__ double lds[SW_REC * NS];
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(SW_THREADS, 1) void k_sweep(S sc, SweepDev d, int p
         double2 e[NE];
 #pragma unroll
         for (int i = 0; i < NE; ++i) e[i] = d.ent[((size_t)k * NE + i) * np + s];
-        const int sl = d.more[(size_t)k * np + s];
+        const int sl = d.more[(size_t)(k - SW_MAXE) * np + s];
         if (TAIL == 1 || sl >= 0) {
           add(sl, e);
         } else {

@@ -45,33 +45,41 @@ constexpr size_t SW_MAX_CNT = (1 << 15) - 1;
 // of nb, each a neighbour's position; out: where a position's result goes.
 // A node with more neighbours beyond the ring than a pass can fetch (a hub of
 // a mesh, of any number) reads those that have no slot from their stored
-// records, slot[] being the bit-inverted place there; never one of its first
+// records, a bit-inverted place there in `more`; never one of its first
 // SW_MAXE entries, which take at most as many of its pass's SW_WIDTH slots.
 // No passes: the nodes or a node's entries are more than the kernel takes,
 // and the caller sweeps by level launches.
 struct SweepPlan {
-  std::vector<int4> pass, head;
-  std::vector<int> far, slot;
+  std::vector<int4> pass, head;  // as SweepDev has them
+  std::vector<int> far, more;
   int npass[2] = {0, 0}, nstep[2] = {0, 0};  // of the forward and the backward sweep
-  int q = SW_MAXE;
+  int q = SW_MAXE;     // the most entries of a node, at least SW_MAXE
   bool spill = false;  // some entries are read from their stored records
 };
+
+// The least steps that the levels with offsets `off` can take (known before
+// the plan).
+inline size_t sweep_least_steps(const std::vector<int>& off) {
+  size_t n = 0;
+  for (size_t l = 0; l + 1 < off.size(); ++l)
+    n += ((size_t)(off[l + 1] - off[l]) + SW_THREADS - 1) / SW_THREADS;
+  return n;
+}
 
 inline SweepPlan sweep_plan(int n, const std::vector<int>& off_f, const std::vector<int>& off_b,
                             const std::vector<size_t>& eptr, const std::vector<int>& nb,
                             const std::vector<int>& out, int ring) {
+  static_assert(SW_MAXE == 5 && SW_MAXE <= SW_WIDTH, "what a head holds; and has slots");
   SweepPlan p;
   const size_t np = 2 * (size_t)n;
   if (np > SW_MAX_POS) return p;
-  for (size_t s = 0; s < np; ++s)
-    if (eptr[s + 1] - eptr[s] > SW_MAX_CNT) return p;
-  std::vector<int> cnt(np);
-  std::vector<char> fetched(np, 0);
-  for (size_t s = 0; s < np; ++s) {
-    cnt[s] = (int)(eptr[s + 1] - eptr[s]);
-    p.q = std::max(p.q, cnt[s]);
-  }
-  p.slot.assign((size_t)p.q * np, sw_zero_slot(ring));
+  size_t q = SW_MAXE;
+  for (size_t s = 0; s < np; ++s) q = std::max(q, eptr[s + 1] - eptr[s]);
+  if (q > SW_MAX_CNT) return p;
+  p.q = (int)q;
+  const int zero = sw_zero_slot(ring);
+  p.head.resize(np);
+  p.more.assign((q - SW_MAXE) * np, zero);
   for (int dir = 0; dir < 2; ++dir) {
     const std::vector<int>& off = dir == 0 ? off_f : off_b;
     const int base = dir == 0 ? 0 : n;  // ring slots count from the sweep's first position
@@ -95,24 +103,28 @@ inline SweepPlan sweep_plan(int n, const std::vector<int>& off_f, const std::vec
           int need = 0;
           for (size_t j = eptr[s]; j < eptr[s + 1]; ++j) need += nb[j] < lim;
           if (cnt_far + need > SW_WIDTH && m > 0) break;
-          for (size_t j = eptr[s]; j < eptr[s + 1]; ++j) {
-            const int o = nb[j];
-            int sl;
+          const int cnt = (int)(eptr[s + 1] - eptr[s]);
+          int sl[SW_MAXE] = {zero, zero, zero, zero, zero};
+          for (int k = 0; k < cnt; ++k) {
+            const int o = nb[eptr[s] + k];
+            int at_slot;
             if (o >= lim) {
-              sl = (o - base) % ring;
+              at_slot = (o - base) % ring;
             } else {
-              fetched[o] = 1;
+              p.head[o].z |= (int)0x80000000;
               if (cnt_far < SW_WIDTH) {
-                sl = ring + (at - at0) % SW_WAVES * SW_WIDTH + cnt_far;
+                at_slot = ring + (at - at0) % SW_WAVES * SW_WIDTH + cnt_far;
                 far[cnt_far++] = o - base;
               } else {
-                sl = ~(o - base);
+                at_slot = ~(o - base);
                 p.spill = true;
               }
             }
-            p.slot[(j - eptr[s]) * np + s] = sl;
+            if (k < SW_MAXE) sl[k] = at_slot;
+            else p.more[(size_t)(k - SW_MAXE) * np + s] = at_slot;
           }
-          mc = std::max(mc, cnt[s]);
+          p.head[s] = make_int4(sl[0] | sl[1] << 16, sl[2] | sl[3] << 16, sl[4] | cnt << 16, out[s]);
+          mc = std::max(mc, cnt);
         }
         p.pass.push_back(make_int4(b, m, step, mc));
         b += m;
@@ -128,13 +140,6 @@ inline SweepPlan sweep_plan(int n, const std::vector<int>& off_f, const std::vec
     }
     p.npass[dir] = (int)p.pass.size() - at0;
     p.nstep[dir] = step + 1;
-  }
-  static_assert(SW_MAXE <= SW_WIDTH, "the entries of the head have slots");
-  p.head.resize(np);
-  for (size_t s = 0; s < np; ++s) {
-    auto sl = [&](int k) { return p.slot[(size_t)k * np + s]; };
-    p.head[s] = make_int4(sl(0) | sl(1) << 16, sl(2) | sl(3) << 16,
-                          sl(4) | cnt[s] << 16 | (fetched[s] ? (int)0x80000000 : 0), out[s]);
   }
   return p;
 }
