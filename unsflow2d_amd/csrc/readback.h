@@ -24,9 +24,9 @@
 #include <memory>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 
+#include "helper_threads.h"
 #include "ufx_internal.h"
 
 namespace ufx {
@@ -166,11 +166,8 @@ static int read_rows(Readback& rb, int device, hipStream_t stream, const double*
   std::thread th[RB_THREADS - 1];
   const int most = (int)std::min<size_t>(
       {RB_THREADS, bytes / RB_SHARE, std::max(1u, std::thread::hardware_concurrency())});
-  int nth = 0;
-  try {
-    for (; nth < most - 1; ++nth) th[nth] = std::thread(help);
-  } catch (const std::system_error&) {  // the ones that started, and this thread, do it
-  }
+  // (the ones that start, and this thread, do it)
+  const int nth = start_threads(th, most - 1, help);
   for (size_t c = 0; c < nch && bad.load() == hipSuccess; ++c) {
     // the slot's last chunk copied out
     while (c >= (size_t)slots && !done[c - slots].load(std::memory_order_acquire))
