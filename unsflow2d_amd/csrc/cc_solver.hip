@@ -766,11 +766,13 @@ int get_field(ufx_cc* x, DevT<R>& d, const std::string& n, double* dst) {
   const std::vector<int>& sto = x->sto_of_ref;
   if (n == "qc" || n == "qold" || n == "res") {
     const double* src = n == "qc" ? d.qc : (n == "qold" ? d.qold : d.res);
-    return read_rows<4>(x->rb, x->device, x->stream, src, x->d_sto, n == "qc" ? ncell : noc, dst);
+    return read_rows<4>(x->rb, x->device, x->stream, src, x->d_sto, sto,
+                        n == "qc" ? ncell : noc, dst);
   }
   if (n == "dt" || n == "la") {
     if (int rc = restore_dtla(x, d)) return rc;
-    return read_rows<1>(x->rb, x->device, x->stream, n == "dt" ? d.dt : d.la, x->d_sto, noc, dst);
+    return read_rows<1>(x->rb, x->device, x->stream, n == "dt" ? d.dt : d.la, x->d_sto, sto, noc,
+                        dst);
   }
   if (n == "qp" || n == "grad" || n == "phi") {
     std::vector<R> rec((size_t)ncell * RW), t((size_t)ncell), gt((size_t)noc * 2);

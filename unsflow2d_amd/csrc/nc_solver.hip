@@ -1152,8 +1152,8 @@ int ufx_nc_get(ufx_nc* x, const char* name, double* dst) {
   // per-vertex arrays (w values each) from storage slots to the reference's
   // vertex numbering
   auto vertex_array = [&](const double* src, int w) -> int {
-    return w == 4 ? read_rows<4>(x->rb, x->device, x->stream, src, x->d_sto, nop, dst)
-                  : read_rows<1>(x->rb, x->device, x->stream, src, x->d_sto, nop, dst);
+    return w == 4 ? read_rows<4>(x->rb, x->device, x->stream, src, x->d_sto, x->sv, nop, dst)
+                  : read_rows<1>(x->rb, x->device, x->stream, src, x->d_sto, x->sv, nop, dst);
   };
   if (n == "qc") return vertex_array(x->d.qc, 4);
   if (n == "qold") {

@@ -25,6 +25,7 @@
 #include <new>
 #include <string>
 #include <thread>
+#include <vector>
 
 #include "helper_threads.h"
 #include "ufx_internal.h"
@@ -109,14 +110,28 @@ inline int read_failed(hipError_t e) {
   return UFX_ERR_HIP;
 }
 
+// Rows map[0] .. map[n - 1] of src (hmap: the map on the host, a permutation of
+// 0 .. n - 1) to dst.
 template <int W>
 static int read_rows(Readback& rb, int device, hipStream_t stream, const double* src, const int* map,
-              size_t n, double* dst) {
+              const std::vector<int>& hmap, size_t n, double* dst) {
   constexpr size_t ROW = W * sizeof(double);
   const size_t bytes = n * ROW;
   if (n == 0) return UFX_OK;
   const DeviceGuard guard(device);
-  if (hipError_t e = rb.reserve(bytes)) return read_failed(e);
+  if (rb.reserve(bytes) != hipSuccess) {
+    // no pinned memory to be had: through the runtime's own, permuted here
+    std::unique_ptr<double[]> t(new (std::nothrow) double[n * W]);
+    if (!t) {
+      set_error("read-back: out of host memory");
+      return UFX_ERR_HIP;
+    }
+    hipError_t e = hipMemcpyAsync(t.get(), src, bytes, hipMemcpyDeviceToHost, stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) return read_failed(e);
+    for (size_t i = 0; i < n; ++i) std::memcpy(dst + i * W, &t[(size_t)hmap[i] * W], ROW);
+    return UFX_OK;
+  }
   auto gather = [&](size_t i0, size_t m, char* to) {
     const size_t th = W == 4 ? 2 * m : m;
     k_gather_rows<W><<<(unsigned)((th + 255) / 256), 256, 0, stream>>>(src, map, i0, m,
