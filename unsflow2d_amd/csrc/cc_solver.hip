@@ -721,8 +721,8 @@ int run_iteration(ufx_cc* x, DevT<R>& d, int iter, int k) {
   // the fused RK3 stages read the start state from qc (no qold copy)
   const bool fused = x->p.timemode == UFX_TIME_RK3 && !visc && !x->p.irs;
   // the last stage of a fused iteration refreshes the next iteration's
-  // primitives itself (not with the diamond-path gradient, whose face pass
-  // reads the records' primitives before the gradient pass copies them in)
+  // primitives itself (not with the diamond-path gradient, which may stop the
+  // iteration and must then leave this one's primitives in the records)
   const bool epi = fused && x->p.grad != UFX_GRAD_GGFC && x->iter_fusion;
   x->qold_stale = fused;
   const bool refresh = !(epi && x->prims_next);

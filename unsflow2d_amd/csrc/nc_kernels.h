@@ -1148,7 +1148,7 @@ __global__ __launch_bounds__(BLK) void k_nc_lusgs_mc(DevNC d, NCFree g, int s0, 
 
 // ---- reference-order sweeps in one workgroup (sweep.h)
 // The LDS ring of the last positions' records (with the area of the stored
-// records beside it 134 KB of a CU's 160 KB); 1.4 % to 3 % of the reads of a
+// records beside it 134 KB of a CU's 160 KB); 2.1 % to 3.5 % of the reads of a
 // 180 000-vertex O-grid lie beyond it.
 constexpr int SW_RING = 1536;
 constexpr int SW_ENTRIES = 5;  // 0.1 % of an O-grid's vertices have more swept neighbours

@@ -18,7 +18,8 @@
 //     density, velocities, pressure and total enthalpy of its new state, so
 //     that their divisions are done once per node and not once per edge --
 //     in an LDS ring of the last SW_RING positions;
-//   - a neighbour further back (a few per cent of the reads) is fetched from
+//   - a neighbour further back (1 to 3 % of the reads on an O-grid of 125 000
+//     vertices, 6 to 10 % on 500 000, a third on two million) is fetched from
 //     its stored record passes ahead into a second LDS area, at a slot that
 //     the host has assigned: inside a pass every read is an LDS read (but for
 //     nodes with more neighbours further back than a pass can fetch);
@@ -35,7 +36,11 @@
 // level launches took 7.2 us each, 4 ms a sweep.  The NC solver on 125 000
 // vertices (1240 steps): 1444 / 1496 us, 1.2 us a step, where one workgroup
 // of 1024 threads with an LDS ring of dq alone, which formed each neighbour's
-// new state again at every edge, took 4350 us.  Half of a step is the
+// new state again at every edge, took 4350 us.  A whole iteration takes 3.0,
+// 12.5 and 61 ms on 125 000, 500 000 and two million vertices (2.4 steps a
+// level there), where that one took 8.6, 25.5 and 71.7; 9.8 and 41.8 ms on
+// 500 000 and two million cells, where the level launches took 37 and 92.
+// Half of a step is the
 // arithmetic of one wave (an NC node is some 600 double precision
 // instructions of four cycles), the rest LDS latency and the barrier; the
 // bytes (about 1.2 KB a node) would take a tenth.  Tried and slower: two
